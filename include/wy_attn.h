@@ -471,12 +471,35 @@ int wy_gdn_chunk_output(const void *q, const int64_t *q_strides, const void *k,
                         void *stream);
 
 /*
- * Gated DeltaNet sequential prefill over a packed varlen batch: sequence b
- * owns tokens [cu_seqlens[b], cu_seqlens[b+1]) of q, k [T, H, key_dim],
- * v, out [T, H, value_dim] (bf16), beta, g [T, H] fp32, and starts from a
- * zero state; its final state goes to state[b] ([B, H, key_dim, value_dim]
- * fp32, unit inner stride).  cu_seqlens [B+1] int32 on the device.  Same
- * step as wy_gdn_recurrent_decode.  Allocates nothing; one launch.
+ * Gated DeltaNet prefill over a packed varlen batch: sequence b owns tokens
+ * [cu_seqlens[b], cu_seqlens[b+1]) of q, k [T, H, key_dim], v, out
+ * [T, H, value_dim] (bf16), beta, g [T, H] fp32, and starts from a zero state;
+ * its final state goes to state[b] ([B, H, key_dim, value_dim] fp32, unit
+ * inner stride).  cu_seqlens [B+1] int32 on the device (NULL: one sequence of
+ * token_num tokens, batch 1).  The recurrence of
+ * wy_gdn_recurrent_decode, formed 32 tokens at a time at fp32 accuracy.
+ * token_num: T; workspace: NULL / 0 bytes, or 16-byte aligned device memory of
+ * at least wy_gdn_prefill_varlen_workspace_bytes(T, H, value_dim) bytes (no
+ * initial contents needed), with which sequences of more than 512 tokens are
+ * cut into segments that run side by side (three launches in place of one; the
+ * results differ in the last bits of the fp32 sums).  Allocates nothing.
+ * Replaces wy_lib::gdn_recurrent_prefill_sequential
+ *   (triton_kernels/gdn_recurrent_prefill.py:1050-1146, kernel :52-143).
+ */
+int wy_gdn_prefill_varlen(const void *q, const int64_t *q_strides, const void *k,
+                          const int64_t *k_strides, const void *v, const int64_t *v_strides,
+                          const float *beta, const int64_t *beta_strides, const float *g,
+                          const int64_t *g_strides, void *out, const int64_t *out_strides,
+                          float *state, const int64_t *state_strides, const int32_t *cu_seqlens,
+                          int token_num, int batch, int num_heads, int key_dim, int value_dim,
+                          float *workspace, int64_t workspace_bytes, void *stream);
+
+/* Workspace size of wy_gdn_prefill_varlen (0: none needed). */
+int64_t wy_gdn_prefill_varlen_workspace_bytes(int token_num, int num_heads, int value_dim);
+
+/*
+ * wy_gdn_prefill_varlen without a workspace: one launch, every sequence walked
+ * from its start.
  * Replaces wy_lib::gdn_recurrent_prefill_sequential
  *   (triton_kernels/gdn_recurrent_prefill.py:1050-1146, kernel :52-143).
  */

@@ -67,6 +67,9 @@ _SIGNATURES = {
     "wy_gdn_recurrent_prefill_sequential": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp,
                                             _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p,
                                             _vp, _i, _i, _i, _i, _vp],
+    "wy_gdn_prefill_varlen": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp,
+                              _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _i, _i, _i, _i, _i, _vp,
+                              _i64, _vp],
     "wy_depthwise_causal_conv4_decode": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp,
                                          _c_i64p, _i, _i, _vp],
     "wy_gdn_qk_norm_gates": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _vp,
@@ -91,7 +94,8 @@ _SIGNATURES = {
 # entry points returning a size (int64) rather than a status
 _SIZE_QUERIES = ("wy_varlen_causal_prefill_workspace_bytes", "wy_gemm_2d_workspace_bytes",
                  "wy_gemm_2d_gate_up_swiglu_workspace_bytes",
-                 "wy_lm_head_argmax_workspace_bytes", "wy_paged_decode_step_noalloc_max_rows",
+                 "wy_lm_head_argmax_workspace_bytes", "wy_gdn_prefill_varlen_workspace_bytes",
+                 "wy_paged_decode_step_noalloc_max_rows",
                  "wy_page_stream_read_waves")
 
 # test hooks returning nothing
@@ -123,7 +127,8 @@ def load() -> ctypes.CDLL:
     lib.wy_build_info.restype = ctypes.c_char_p
     for fn in (lib.wy_varlen_causal_prefill_workspace_bytes, lib.wy_gemm_2d_workspace_bytes,
                lib.wy_gemm_2d_gate_up_swiglu_workspace_bytes,
-               lib.wy_lm_head_argmax_workspace_bytes):
+               lib.wy_lm_head_argmax_workspace_bytes,
+               lib.wy_gdn_prefill_varlen_workspace_bytes):
         fn.argtypes = [_i, _i, _i]
         fn.restype = ctypes.c_int64
     for fn in (lib.wy_paged_decode_step_noalloc_max_rows, lib.wy_page_stream_read_waves):

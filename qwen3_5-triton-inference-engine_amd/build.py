@@ -21,8 +21,8 @@ OBJ_DIR = PKG_DIR / "_build"
 ARCH = os.environ.get("WY_OFFLOAD_ARCH", "gfx950")
 
 SOURCES = ["capi.hip", "kv_cache.hip", "rope_gate.hip", "rmsnorm.hip", "decode.hip", "prefill.hip",
-           "prefill_direct.hip", "prefill_short.hip", "gemm.hip", "gdn.hip", "gdn_block.hip", "gdn_chunk.hip",
-           "model_ops.hip"]
+           "prefill_direct.hip", "prefill_short.hip", "gemm.hip", "gdn.hip", "gdn_block.hip",
+           "gdn_chunk.hip", "gdn_scan.hip", "model_ops.hip"]
 
 # Per-source extra flags.  The direct-launch prefill variants keep their MFMA
 # accumulators in VGPRs (faster there; the queue variants in prefill.hip are

@@ -1,5 +1,5 @@
-// Device code shared by the Gated DeltaNet kernels (gdn.hip, gdn_block.hip):
-// the lane layout of a state block and one delta-rule step, so the fused
+// Code shared by the Gated DeltaNet kernels (gdn.hip, gdn_block.hip, gdn_scan.hip):
+// the argument checks, the decode kernels' lane layout of a state block and one delta-rule step, so the fused
 // decode block and the standalone recurrence run identical arithmetic.
 //
 // One wavefront owns 16 value columns of one (sequence, head) with all
@@ -85,101 +85,20 @@ __device__ __forceinline__ void store4(bf16_t *p, int64_t stride, const float (&
   }
 }
 
-// One token's inputs for one lane (NC value columns).
-template <int NC>
-struct TokenInT {
-  float k[kRows], q[kRows], v[NC];
+// One token's inputs for one lane.
+struct TokenIn {
+  float k[kRows], q[kRows], v[kCols];
   float g, beta;
 };
-using TokenIn = TokenInT<kCols>;
 
-template <bool kContig, int NC = kCols>
+template <bool kContig>
 __device__ __forceinline__ void load_token(const GdnArgs &a, int64_t t, int h, int kg, int col,
-                                           TokenInT<NC> &in) {
+                                           TokenIn &in) {
   load8<kContig>(a.k + t * a.k_t + h * a.k_h + kg * kRows * a.k_d, a.k_d, in.k);
   load8<kContig>(a.q + t * a.q_t + h * a.q_h + kg * kRows * a.q_d, a.q_d, in.q);
-  const bf16_t *vp = a.v + t * a.v_t + h * a.v_h + col * a.v_d;
-  if constexpr (NC == kCols)
-    load4<kContig>(vp, a.v_d, in.v);
-  else
-#pragma unroll
-    for (int e = 0; e < NC; ++e) in.v[e] = bf16_to_f32(vp[e * a.v_d]);
+  load4<kContig>(a.v + t * a.v_t + h * a.v_h + col * a.v_d, a.v_d, in.v);
   in.g = a.g[t * a.g_t + h * a.g_h];
   in.beta = a.beta[t * a.beta_t + h * a.beta_h];
-}
-
-// One token's inputs as loaded (bf16 bits, fp32 g / beta), for prefetching:
-// the bf16 -> fp32 unpack happens at the step (unpack_token), so the loads of
-// later tokens stay in flight while a step runs.  g and beta are read through
-// VGPR addresses: vector loads complete in order, so waiting for this token's
-// values does not wait for the prefetches issued after them (scalar loads
-// return out of order and a wait on one is a wait on all).
-template <int NC>
-struct TokenRaw {
-  u32x4_t k, q;
-  uint32_t v[NC == kCols ? 2 : NC];
-  float g, beta;
-};
-typedef const __attribute__((address_space(1))) float gfloat_t;
-
-template <bool kContig, int NC>
-__device__ __forceinline__ void load_token_raw(const GdnArgs &a, int64_t t, int h, int kg, int col,
-                                               TokenRaw<NC> &r) {
-  const bf16_t *kp = a.k + t * a.k_t + h * a.k_h + kg * kRows * a.k_d;
-  const bf16_t *qp = a.q + t * a.q_t + h * a.q_h + kg * kRows * a.q_d;
-  const bf16_t *vp = a.v + t * a.v_t + h * a.v_h + col * a.v_d;
-  if constexpr (kContig) {
-    r.k = ld16(kp);
-    r.q = ld16(qp);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      r.k[e] = uint32_t(kp[2 * e * a.k_d]) | (uint32_t(kp[(2 * e + 1) * a.k_d]) << 16);
-      r.q[e] = uint32_t(qp[2 * e * a.q_d]) | (uint32_t(qp[(2 * e + 1) * a.q_d]) << 16);
-    }
-  }
-  if constexpr (NC == kCols) {
-    if constexpr (kContig) {
-      const u32x2_t w = *reinterpret_cast<const u32x2_t *>(vp);
-      r.v[0] = w[0];
-      r.v[1] = w[1];
-    } else {
-      r.v[0] = uint32_t(vp[0]) | (uint32_t(vp[a.v_d]) << 16);
-      r.v[1] = uint32_t(vp[2 * a.v_d]) | (uint32_t(vp[3 * a.v_d]) << 16);
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < NC; ++e) r.v[e] = uint32_t(vp[e * a.v_d]);
-  }
-  gfloat_t *gp = (gfloat_t *)(a.g + t * a.g_t + h * a.g_h);
-  gfloat_t *bp = (gfloat_t *)(a.beta + t * a.beta_t + h * a.beta_h);
-  asm volatile("" : "+v"(gp), "+v"(bp));
-  r.g = *gp;
-  r.beta = *bp;
-}
-
-template <int NC>
-__device__ __forceinline__ TokenInT<NC> unpack_token(const TokenRaw<NC> &r) {
-  TokenInT<NC> in;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    in.k[2 * e] = bf16_lo(r.k[e]);
-    in.k[2 * e + 1] = bf16_hi(r.k[e]);
-    in.q[2 * e] = bf16_lo(r.q[e]);
-    in.q[2 * e + 1] = bf16_hi(r.q[e]);
-  }
-  if constexpr (NC == kCols) {
-    in.v[0] = bf16_lo(r.v[0]);
-    in.v[1] = bf16_hi(r.v[0]);
-    in.v[2] = bf16_lo(r.v[1]);
-    in.v[3] = bf16_hi(r.v[1]);
-  } else {
-#pragma unroll
-    for (int e = 0; e < NC; ++e) in.v[e] = bf16_lo(r.v[e]);
-  }
-  in.g = r.g;
-  in.beta = r.beta;
-  return in;
 }
 
 // One delta-rule step on the lane's 8 x 4 block of S; returns the lane's 4
@@ -221,51 +140,41 @@ __device__ __forceinline__ void gdn_step(float (&s)[kRows][kCols], const TokenIn
     for (int j = 0; j < kCols; ++j) s[i][j] = __fmaf_rn(in.k[i], delta[j], s[i][j]);
 }
 
-// The same step on a lazily decayed state: the true state is c * s.  The
-// decay only scales c; the reductions use s and are scaled by c, and the
-// rank-1 update adds k (delta / c).  When c drops below 2^-32 it is folded
-// into s first (c = 0, a full decay, clears s).  This saves the per-element
-// decay multiply of every token (3 instead of 4 VALU ops per state element);
-// the values agree with gdn_step to fp32 rounding.
-template <int NC = kCols>
-__device__ __forceinline__ void gdn_step_scaled(float (&s)[kRows][NC], float &c,
-                                                const TokenInT<NC> &in, float (&o)[NC]) {
-  c *= __expf(in.g);
-  if (c < 0x1p-32f) {  // uniform: c depends on the token only
-#pragma unroll
-    for (int i = 0; i < kRows; ++i)
-#pragma unroll
-      for (int j = 0; j < NC; ++j) s[i][j] *= c;
-    c = 1.f;
-  }
-  float mem[NC], qs[NC], qk = 0.f;
-#pragma unroll
-  for (int j = 0; j < NC; ++j) {
-    mem[j] = 0.f;
-    qs[j] = 0.f;
-  }
-#pragma unroll
-  for (int i = 0; i < kRows; ++i) {
-    qk = __fmaf_rn(in.q[i], in.k[i], qk);
-#pragma unroll
-    for (int j = 0; j < NC; ++j) {
-      mem[j] = __fmaf_rn(in.k[i], s[i][j], mem[j]);
-      qs[j] = __fmaf_rn(in.q[i], s[i][j], qs[j]);
-    }
-  }
-  qk = sum16(qk);
-  const float inv_c = __builtin_amdgcn_rcpf(c);  // v_rcp_f32 (1 ulp): only scales the update
-  float dsc[NC];
-#pragma unroll
-  for (int j = 0; j < NC; ++j) {
-    const float delta = in.beta * (in.v[j] - c * sum16(mem[j]));
-    o[j] = __fmaf_rn(qk, delta, c * sum16(qs[j]));
-    dsc[j] = delta * inv_c;
-  }
-#pragma unroll
-  for (int i = 0; i < kRows; ++i)
-#pragma unroll
-    for (int j = 0; j < NC; ++j) s[i][j] = __fmaf_rn(in.k[i], dsc[j], s[i][j]);
+// Shared argument checks; returns WY_OK and fills a, or an error code.
+inline int gdn_setup(GdnArgs &a, bool &contig, const void *q, const int64_t *qs, const void *k,
+              const int64_t *ks, const void *v, const int64_t *vs, const float *beta,
+              const int64_t *bs, const float *g, const int64_t *gs, void *out,
+              const int64_t *os, float *state, const int64_t *ss, int heads, int key_dim,
+              int value_dim) {
+  if (!q || !qs || !k || !ks || !v || !vs || !beta || !bs || !g || !gs || !out || !os ||
+      !state || !ss)
+    return WY_E_NULL;
+  if (heads <= 0 || key_dim <= 0 || value_dim <= 0) return WY_E_SHAPE;
+  if (key_dim != kDK || value_dim % 128 != 0) return WY_E_UNSUPPORTED;
+  if (ss[3] != 1 || ss[2] % 4 || ss[1] % 4 || ss[0] % 4 || !wyh::aligned16(state))
+    return WY_E_LAYOUT;
+  a = GdnArgs{};
+  a.q = static_cast<const bf16_t *>(q);
+  a.k = static_cast<const bf16_t *>(k);
+  a.v = static_cast<const bf16_t *>(v);
+  a.q_t = qs[0]; a.q_h = qs[1]; a.q_d = qs[2];
+  a.k_t = ks[0]; a.k_h = ks[1]; a.k_d = ks[2];
+  a.v_t = vs[0]; a.v_h = vs[1]; a.v_d = vs[2];
+  a.beta = beta; a.beta_t = bs[0]; a.beta_h = bs[1];
+  a.g = g; a.g_t = gs[0]; a.g_h = gs[1];
+  a.out = static_cast<bf16_t *>(out);
+  a.o_t = os[0]; a.o_h = os[1]; a.o_d = os[2];
+  a.state = state;
+  a.s_b = ss[0]; a.s_h = ss[1]; a.s_k = ss[2]; a.s_v = ss[3];
+  a.heads = heads;
+  a.dv = value_dim;
+  // 16-byte q/k rows (8 bf16 per lane) and 8-byte v / out quads
+  contig = qs[2] == 1 && ks[2] == 1 && vs[2] == 1 && os[2] == 1 && qs[0] % 8 == 0 &&
+           qs[1] % 8 == 0 && ks[0] % 8 == 0 && ks[1] % 8 == 0 && wyh::aligned16(q) &&
+           wyh::aligned16(k) && vs[0] % 4 == 0 && vs[1] % 4 == 0 && os[0] % 4 == 0 &&
+           os[1] % 4 == 0 && (reinterpret_cast<uintptr_t>(v) & 7u) == 0 &&
+           (reinterpret_cast<uintptr_t>(out) & 7u) == 0;
+  return WY_OK;
 }
 
 }  // namespace gdn

@@ -4,8 +4,9 @@ Drop-in for the recurrent ops of ``triton_kernels/gdn_recurrent_prefill.py``:
 same op names ``wy_lib::gdn_recurrent_decode`` and
 ``wy_lib::gdn_recurrent_prefill_sequential``, schemas, assertions and
 returned layouts (reference :1050-1146, :1185-1260), plus the
-``call_*_triton`` wrappers (:1174-1182, :1274-1282).  Both run one launch of
-``csrc/gdn.hip``; there is no CPU path.
+``call_*_triton`` wrappers (:1174-1182, :1274-1282).  Decode is one launch of
+``csrc/gdn.hip``, prefill one to three of ``csrc/gdn_scan.hip``; there is no
+CPU path.
 """
 
 from __future__ import annotations
@@ -40,6 +41,20 @@ def _tensor_args(q, k, v, beta, g, out, state):
     )
 
 
+def _prefill(q, k, v, beta, g, out, state, cu_seqlens):
+    """The packed prefill into ``out`` and ``state``.  The workspace (segment
+    states of sequences over 512 tokens) lives for this call."""
+    token_num, num_heads, key_dim = q.shape
+    value_dim = v.shape[-1]
+    nbytes = _lib.load().wy_gdn_prefill_varlen_workspace_bytes(token_num, num_heads, value_dim)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+    _lib.call(
+        "wy_gdn_prefill_varlen", *_tensor_args(q, k, v, beta, g, out, state),
+        _lib.ptr(cu_seqlens), token_num, state.shape[0], num_heads, key_dim, value_dim,
+        _lib.ptr(ws), nbytes, _lib.stream(q.device),
+    )
+
+
 @torch.library.custom_op(
     "wy_lib::gdn_recurrent_prefill_sequential", mutates_args=(), device_types="cuda"
 )
@@ -60,26 +75,19 @@ def gdn_recurrent_prefill_sequential(
     token_num, num_heads, key_dim = q.shape
     value_dim = v.shape[-1]
     assert token_num > 0 and num_heads > 0
-    if cu_seqlens is None:
-        cu_seqlens = torch.tensor([0, token_num], dtype=torch.int32, device=q.device)
-        squeeze_state = True
-    else:
+    if cu_seqlens is not None:
         assert cu_seqlens.dtype == torch.int32 and cu_seqlens.ndim == 1
         assert int(cu_seqlens[-1]) == token_num, (
             f"cu_seqlens[-1]={int(cu_seqlens[-1])} does not match the packed token count "
             f"{token_num}"
         )
         cu_seqlens = cu_seqlens.contiguous()
-        squeeze_state = False
-    batch = cu_seqlens.numel() - 1
+    batch = 1 if cu_seqlens is None else cu_seqlens.numel() - 1
     out = torch.empty_like(v)
     state = torch.empty((batch, num_heads, key_dim, value_dim), dtype=torch.float32,
                         device=q.device)
-    _lib.call(
-        "wy_gdn_recurrent_prefill_sequential", *_tensor_args(q, k, v, beta, g, out, state),
-        _lib.ptr(cu_seqlens), batch, num_heads, key_dim, value_dim, _lib.stream(q.device),
-    )
-    return out, (state[0] if squeeze_state else state)
+    _prefill(q, k, v, beta, g, out, state, cu_seqlens)
+    return out, (state[0] if cu_seqlens is None else state)
 
 
 @gdn_recurrent_prefill_sequential.register_fake
@@ -104,10 +112,7 @@ def gdn_prefill_sequential_into(q, k, v, beta, g, cu_seqlens, state):
     assert state.dtype == torch.float32
     assert state.shape == (batch, num_heads, key_dim, value_dim)
     out = torch.empty_like(v)
-    _lib.call(
-        "wy_gdn_recurrent_prefill_sequential", *_tensor_args(q, k, v, beta, g, out, state),
-        _lib.ptr(cu_seqlens), batch, num_heads, key_dim, value_dim, _lib.stream(q.device),
-    )
+    _prefill(q, k, v, beta, g, out, state, cu_seqlens)
     return out
 
 
@@ -295,8 +300,7 @@ def call_gdn_chunk_output_triton(q, k, delta, g_cumsum, chunk_state):
 
 
 def call_gdn_recurrent_prefill_chunked_triton(q, k, v, beta, g):
-    """One prompt through the three chunk launches: ``(out [T, H, DV] bf16,
-    final_state [H, DK, DV] fp32)`` (reference gdn_recurrent_prefill.py:1026-1048)."""
-    w, u_base, g_cumsum = gdn_chunk_prepare_wy(k, v, beta, g)
-    delta, chunk_state, final_state = gdn_chunk_state(k, w, u_base, g_cumsum)
-    return gdn_chunk_output(q, k, delta, g_cumsum, chunk_state), final_state
+    """One prompt: ``(out [T, H, DV] bf16, final_state [H, DK, DV] fp32)``, the
+    result of the chunk ops above (reference gdn_recurrent_prefill.py:1026-1048)
+    by the packed prefill's kernels, which form no intermediate tensors."""
+    return gdn_recurrent_prefill_sequential(q, k, v, beta, g)

@@ -1,0 +1,148 @@
+"""The chunked varlen GDN prefill (csrc/gdn_scan.hip) where it can go wrong:
+edges of the 32-token chunks, the 64-token groups and the 512-token segments,
+strides without the 16-byte form, values that are not finite, graph replays.
+Reference: the token-by-token recurrence in float64."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+H, D = 2, 128
+SEG = 512
+
+
+def inputs(T, dev, seed, decay=1.0):
+    gen = torch.Generator().manual_seed(seed)
+    r = lambda *s: torch.randn(*s, generator=gen)  # noqa: E731
+    q = torch.nn.functional.normalize(r(T, H, D), dim=-1) * D ** -0.5
+    k = torch.nn.functional.normalize(r(T, H, D), dim=-1)
+    g = -torch.nn.functional.softplus(r(T, H)) * decay
+    return [x.to(dev) for x in (q.bfloat16(), k.bfloat16(), r(T, H, D).bfloat16(),
+                                torch.sigmoid(r(T, H)), g)]
+
+
+def recurrence64(q, k, v, beta, g, lens):
+    outs, states, o = [], [], 0
+    q, k, v, beta, g = (x.double() for x in (q, k, v, beta, g))
+    for n in lens:
+        s = torch.zeros(H, D, D, dtype=torch.float64, device=q.device)
+        for t in range(o, o + n):
+            s = s * torch.exp(g[t])[:, None, None]
+            d = beta[t][:, None] * (v[t] - (k[t][:, :, None] * s).sum(1))
+            s = s + k[t][:, :, None] * d[:, None, :]
+            outs.append((q[t][:, :, None] * s).sum(1))
+        states.append(s)
+        o += n
+    return torch.stack(outs), torch.stack(states)
+
+
+def cu_of(lens, dev):
+    return torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32,
+                        device=dev)
+
+
+def rel(x, y):
+    return float((x.double() - y).norm() / y.norm())
+
+
+# decay 0.003: a memory of hundreds of tokens, so that segments feel each other
+@pytest.mark.parametrize("lens, decay", [
+    ([31, 32, 33], 1.0), ([63, 64, 65, 1], 0.05), ([SEG - 1, SEG, SEG + 1], 0.003),
+    ([2 * SEG + 33, 5, 3 * SEG], 0.003), ([40], 30.0)])
+def test_lengths_vs_recurrence(pkg, dev, lens, decay):
+    args = inputs(sum(lens), dev, 7 + sum(lens), decay)
+    out, st = pkg.gdn_recurrent_prefill_sequential(*args, cu_of(lens, dev))
+    o64, s64 = recurrence64(*args, lens)
+    # out: one bf16 rounding (2^-9 at most, 2^-9.2 rms); state: fp32 sums over
+    # the memory's tokens, measured at most 3.4e-7 (the token-by-token fp32
+    # kernel it replaced: 1.3e-6)
+    assert rel(out, o64) < 2 ** -9
+    assert rel(st, s64) < 1e-6
+    # the same bits alone as in the batch
+    o = 0
+    for b, n in enumerate(lens):
+        o1, s1 = pkg.gdn_recurrent_prefill_sequential(*(x[o:o + n] for x in args))
+        assert torch.equal(s1, st[b]) and torch.equal(o1, out[o:o + n])
+        o += n
+
+
+@pytest.mark.parametrize("T", [33, SEG + 70])
+def test_other_strides_same_bits(pkg, dev, T):
+    q, k, v, beta, g = inputs(T, dev, T)
+
+    def spread(x):
+        buf = torch.zeros(*x.shape[:-1], 2 * x.shape[-1], dtype=x.dtype, device=dev)
+        buf[..., ::2] = x
+        return buf[..., ::2]
+
+    want = pkg.gdn_recurrent_prefill_sequential(q, k, v, beta, g)
+    heads_first = [x.transpose(0, 1).contiguous().transpose(0, 1) for x in (q, k, v, beta, g)]
+    wide = torch.cat([q, k, v], -1)
+    views = [wide[..., :D], wide[..., D:2 * D], wide[..., 2 * D:], beta, g]
+    for args in ([spread(q), spread(k), spread(v), spread(beta), spread(g)], heads_first, views):
+        got = pkg.gdn_recurrent_prefill_sequential(*args)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("what", ["v", "k", "q", "beta", "g"])
+@pytest.mark.parametrize("t", [0, 40, SEG + 3])
+def test_nan_stays_behind_its_token(pkg, dev, what, t):
+    """A NaN at token t reaches no earlier token and no other sequence."""
+    T = SEG + 64
+    args = dict(zip(("q", "k", "v", "beta", "g"), inputs(2 * T, dev, 3, 0.1)))
+    cu = cu_of([T, T], dev)
+    want, _ = pkg.gdn_recurrent_prefill_sequential(*args.values(), cu)
+    x = args[what].clone()
+    if x.ndim == 3:
+        x[t, 0, 5] = float("nan")
+    else:
+        x[t, 0] = float("nan")
+    args[what] = x
+    out, st = pkg.gdn_recurrent_prefill_sequential(*args.values(), cu)
+    assert torch.equal(out[:t], want[:t]) and torch.equal(out[T:], want[T:])
+    assert torch.equal(out[:, 1], want[:, 1]) and torch.isfinite(st[:, 1]).all()
+    bad = torch.isnan(out[:T, 0].float())
+    if what == "q":      # the token's own output only
+        assert bad[t].all() and bad.sum() == D and torch.isfinite(st).all()
+    elif what == "v":    # that column from the token on
+        assert bad[t:, 5].all() and bad.sum() == T - t
+        assert torch.isnan(st[0, 0, :, 5]).all() and torch.isfinite(st[0, 0, :, :5]).all()
+    else:
+        assert bad[t:].all() and torch.isnan(st[0, 0]).all()
+
+
+def test_full_decay_and_growth(pkg, dev):
+    """g = -inf clears the state; g > 0 grows it."""
+    T = 100
+    q, k, v, beta, g = inputs(T, dev, 11, 0.2)
+    g[37] = -float("inf")
+    g[64] = -1e30
+    g[70:75] = 0.5
+    out, st = pkg.gdn_recurrent_prefill_sequential(q, k, v, beta, g)
+    o64, s64 = recurrence64(q, k, v, beta, g, [T])
+    assert rel(out, o64) < 2 ** -9 and rel(st, s64[0]) < 1e-6
+
+
+def test_graph_replays_and_other_stream(pkg, dev):
+    lens = [SEG + 40, 77]
+    args = inputs(sum(lens), dev, 5, 0.05)
+    cu = cu_of(lens, dev)
+    st = torch.zeros(2, H, D, D, device=dev)
+    into = pkg.gdn_recurrent_prefill.gdn_prefill_sequential_into
+    want, want_st = into(*args, cu, st).clone(), st.clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        into(*args, cu, st)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = into(*args, cu, st)
+    for _ in range(4):
+        out.zero_()
+        st.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(st, want_st)
+        torch.randn(1 << 20, device=dev).sum()
