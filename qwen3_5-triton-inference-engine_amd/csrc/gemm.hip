@@ -153,11 +153,20 @@ __device__ __forceinline__ void gate_up_epilogue(const f32x4v_t (&red)[kNW][kMT 
 //      of the [M, 2N] projection, equal to the plain GEMM followed by
 //      swiglu_kernel whenever the plain GEMM's plan matches (same waves and
 //      K split; 2N >= 4096).
-template <int kNW, int kMT, int kNT, int kPro = 0, int kEpi = 0>
+//
+// kTwo: the first `over` workgroups sum one 16-column tile more, behind the
+// columns of the grid.  A block or two past a whole round of the CUs as
+// workgroups of their own make one CU read twice what the others do, and a CU
+// takes about 1.8 us for 64 KiB ([8224, 1024], 257 blocks: 6.8 us against 5.4
+// for 8192 at M = 1, 9.9 against 7.0 at M = 32, 16.6 against 9.9 at M = 64;
+// with the tiles on the first workgroups 6.3, 8.1 and 11.8.  A whole block as
+// their second: 7.2 and 9.2.  K slices of it on sixteen extra waves, merged
+// through memory: 7.8 and 10.9).
+template <int kNW, int kMT, int kNT, int kPro = 0, int kEpi = 0, bool kTwo = false>
 __global__ __launch_bounds__(64 * kNW) void gemm_skinny_kernel(
     const bf16_t *__restrict__ x, int64_t xs0, const bf16_t *__restrict__ w, int64_t ws0,
     bf16_t *__restrict__ y, int64_t ys0, int M, int N, int K, float *__restrict__ part,
-    int32_t *__restrict__ cnt, const ProArgs pro) {
+    int32_t *__restrict__ cnt, const ProArgs pro, int over) {
   // kMT = ceil(M / 16) tiles of 16 rows, kNT tiles of 16 columns per
   // workgroup (each x load feeds kNT MFMAs); every load of a 4-step batch is
   // issued before the first MFMA consumes one, so a wave waits for memory once
@@ -172,6 +181,7 @@ __global__ __launch_bounds__(64 * kNW) void gemm_skinny_kernel(
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   static_assert(kEpi == 0 || kNT == 2, "gate/up pairs need two column tiles");
+  static_assert(!kTwo || (kPro == 0 && kEpi == 0), "plain GEMM");
   const int n0 = blockIdx.x * 16 * (kEpi == 1 ? 1 : kNT);
   const int n_split = int(gridDim.y);
   const int ks = K / n_split;  // a multiple of 32 * kNW (host)
@@ -193,103 +203,223 @@ __global__ __launch_bounds__(64 * kNW) void gemm_skinny_kernel(
     xok[mt] = row < M;
     xp[mt] = x + int64_t(xok[mt] ? row : 0) * xs0 + kb + 8 * g;
   }
-  // K runs in batches of four 32-wide steps (all loads of a batch issued
-  // before its first MFMA), then one batch of the remaining kc % 128 steps,
-  // loaded together as well.  The first full batch's W rows are requested
-  // before the A prologue, which does not need them.
+  // K runs in batches of four 32-wide steps and one of the remaining kc % 128.
   const int nfull = kc >> 7, rem = (kc & 127) >> 5;
-  u32x4_t w_first[4][kNT];
-  if (nfull > 0) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int nt = 0; nt < kNT; ++nt) w_first[j][nt] = ld16(wp[nt] + 32 * j);
-  }
+  // A prologue's per-row state: rsigma and the residual row
+  __shared__ float rs_lds[kPro == 1 ? kSkinnyMaxM : 1];
   float rsr[kMT];
   const bf16_t *rp[kMT];
   const bf16_t *nwp = nullptr;
   if constexpr (kPro == 1) {
-    // rsigma of every row: 32 lanes per row, lane l summing the 8-element
-    // chunks (32 kk + l) * 8 in order, then the xor tree (rms_rsigma)
-    __shared__ float rs_lds[kSkinnyMaxM];
-    const int l32 = threadIdx.x & 31;
-    const bool write_x = pro.xout && blockIdx.x == 0 && blockIdx.y == 0;
-    for (int row = threadIdx.x >> 5; row < M; row += 2 * kNW) {
-      const bf16_t *hr = x + int64_t(row) * xs0;
-      const bf16_t *rr = pro.res ? pro.res + int64_t(row) * pro.res0 : nullptr;
-      float ss = 0.f;
-      for (int kk = 0; kk < K / 256; ++kk) {
-        const int c = (32 * kk + l32) * 8;
-        u32x4_t t = ld16(hr + c);
-        if (rr) t = add_bf16x8(t, ld16(rr + c));
-        if (write_x) st16(pro.xout + int64_t(row) * pro.xo0 + c, t);
-        ss = rms_acc8(t, ss);
-      }
-      const float rs = rms_rsigma(ss, K, pro.eps);
-      if (l32 == 0) rs_lds[row] = rs;
-    }
-    __syncthreads();
 #pragma unroll
     for (int mt = 0; mt < kMT; ++mt) {
       const int row = mt * 16 + (lane & 15);
-      rsr[mt] = xok[mt] ? rs_lds[row] : 0.f;
       rp[mt] = pro.res ? pro.res + int64_t(xok[mt] ? row : 0) * pro.res0 + kb + 8 * g : nullptr;
     }
     nwp = pro.nw + kb + 8 * g;
   }
-  // the A operand of rows tile mt at k offset kk (relative to kb + 8 g)
-  auto load_a = [&](int mt, int kk) -> u32x4_t {
-    u32x4_t v = ld16(xp[mt] + kk);
-    if constexpr (kPro == 1) {
-      if (rp[mt]) v = add_bf16x8(v, ld16(rp[mt] + kk));
-      v = norm_bf16x8(v, rsr[mt], ld16(nwp + kk));
-    } else if constexpr (kPro == 2) {
-      v = swiglu_bf16x8(v, ld16(xp[mt] + pro.up_off + kk));
-    }
-    return v;
-  };
+  const bool write_x = kPro == 1 && pro.xout && blockIdx.x == 0 && blockIdx.y == 0;
   f32x4v_t acc[kMT][kNT];
 #pragma unroll
   for (int mt = 0; mt < kMT; ++mt)
 #pragma unroll
     for (int nt = 0; nt < kNT; ++nt) acc[mt][nt] = f32x4v_t{0.f, 0.f, 0.f, 0.f};
-  auto step = [&](const u32x4_t (&wv)[kNT], u32x4_t xv, int mt) {
-    if (!xok[mt]) xv = u32x4_t{0u, 0u, 0u, 0u};
+  // one 32-wide k-step of row tile mt; the A operand from what was loaded for it
+  struct RawA {
+    u32x4_t x, r;   // x and the residual (kPro 1) or the up half (kPro 2)
+  };
+  auto load_raw = [&](int mt, int kk) {
+    RawA a;
+    a.x = ld16(xp[mt] + kk);
+    if constexpr (kPro == 1) {
+      a.r = u32x4_t{0u, 0u, 0u, 0u};
+      if (rp[mt]) a.r = ld16(rp[mt] + kk);
+    } else if constexpr (kPro == 2) {
+      a.r = ld16(xp[mt] + pro.up_off + kk);
+    }
+    return a;
+  };
+  auto operand = [&](const RawA &a, u32x4_t nw8, int mt) {
+    u32x4_t xv = a.x;
+    if constexpr (kPro == 1) {
+      if (rp[mt]) xv = add_bf16x8(xv, a.r);
+      xv = norm_bf16x8(xv, rsr[mt], nw8);
+    } else if constexpr (kPro == 2) {
+      xv = swiglu_bf16x8(xv, a.r);
+    }
+    return xok[mt] ? xv : u32x4_t{0u, 0u, 0u, 0u};
+  };
+  auto step = [&](f32x4v_t (&ac)[kMT][kNT], const u32x4_t (&wv)[kNT], u32x4_t xv, int mt) {
 #pragma unroll
     for (int nt = 0; nt < kNT; ++nt)
-      acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-          __builtin_bit_cast(bf16x8_t, xv), __builtin_bit_cast(bf16x8_t, wv[nt]), acc[mt][nt], 0,
+      ac[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+          __builtin_bit_cast(bf16x8_t, xv), __builtin_bit_cast(bf16x8_t, wv[nt]), ac[mt][nt], 0,
           0, 0);
   };
-  // R steps from k: x loads, then the MFMAs over the given W rows
-  auto batch = [&](auto steps, const u32x4_t (&wv)[decltype(steps)::value][kNT], int k) {
-    constexpr int R = decltype(steps)::value;
-    u32x4_t xv[kMT][R];
+  const int n2 = int(gridDim.x) * 16 * kNT + int(blockIdx.x) * 16;   // the tile more
+  const bool two = kTwo && int(blockIdx.x) < over;
+  f32x4v_t acc2[kTwo ? kMT : 1];
+  if constexpr (kTwo) {
 #pragma unroll
-    for (int mt = 0; mt < kMT; ++mt)
+    for (int mt = 0; mt < kMT; ++mt) acc2[mt] = f32x4v_t{0.f, 0.f, 0.f, 0.f};
+  }
+  auto load_tile2 = [&](auto &wv2, int k) {
+    const bf16_t *p2 = w + int64_t(min(n2 + (lane & 15), N - 1)) * ws0 + kb + 8 * g + k;
 #pragma unroll
-      for (int j = 0; j < R; ++j) xv[mt][j] = load_a(mt, k + 32 * j);
+    for (int j = 0; j < int(sizeof(wv2) / sizeof(wv2[0])); ++j) wv2[j] = ld16(p2 + 32 * j);
+  };
+  auto step2 = [&](u32x4_t wv2, u32x4_t xv, int mt) {
+    acc2[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+        __builtin_bit_cast(bf16x8_t, xv), __builtin_bit_cast(bf16x8_t, wv2), acc2[mt], 0, 0, 0);
+  };
+  auto finish_rs = [&]() {   // rsigma of this lane's rows
+#pragma unroll
+    for (int mt = 0; mt < kMT; ++mt) rsr[mt] = xok[mt] ? rs_lds[mt * 16 + (lane & 15)] : 0.f;
+  };
+  // A slice of one to two batches (kc 128 .. 224, most of the model's decode
+  // projections) in one memory round trip: everything the wave will read is
+  // requested before the first value is used, the small operands first.  Loads
+  // complete in order, so what the RMSNorm needs must not queue behind the
+  // weight rows, which come from HBM.  Against W rows first and the A operand
+  // read behind the prologue's barrier: [7168, 1024] plain 7.2 -> 6.8 us at M =
+  // 32, with the RMSNorm 7.5 -> 7.0 at M = 1 and 9.4 -> 7.9 at M = 16.  Same
+  // operations in the same order as below.
+  constexpr int kOnceRows = 2 * kNW;   // rows the prologue norms in one pass
+  auto once = [&](auto steps) {
+    constexpr int R = decltype(steps)::value;   // k-steps
+    const int l32 = threadIdx.x & 31, prow = threadIdx.x >> 5;
+    u32x4_t nx[4], nr[4];
+    const int nkk = K / 256;
+    if constexpr (kPro == 1) {
+      const bf16_t *hr = x + int64_t(min(prow, M - 1)) * xs0 + 8 * l32;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) nx[kk] = ld16(hr + 256 * min(kk, nkk - 1));
+      if (pro.res) {
+        const bf16_t *rr = pro.res + int64_t(min(prow, M - 1)) * pro.res0 + 8 * l32;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) nr[kk] = ld16(rr + 256 * min(kk, nkk - 1));
+      }
+    }
+    RawA av[kMT][R];
+    u32x4_t nv[R], wv[R][kNT];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+#pragma unroll
+      for (int mt = 0; mt < kMT; ++mt) av[mt][j] = load_raw(mt, 32 * j);
+      nv[j] = u32x4_t{0u, 0u, 0u, 0u};
+      if constexpr (kPro == 1) nv[j] = ld16(nwp + 32 * j);
+    }
 #pragma unroll
     for (int j = 0; j < R; ++j)
 #pragma unroll
-      for (int mt = 0; mt < kMT; ++mt) step(wv[j], xv[mt][j], mt);
-  };
-  auto load_batch = [&](auto steps, int k) {
-    constexpr int R = decltype(steps)::value;
-    u32x4_t wv[R][kNT];
+      for (int nt = 0; nt < kNT; ++nt) wv[j][nt] = ld16(wp[nt] + 32 * j);
+    u32x4_t wv2[kTwo ? R : 1];
+    if constexpr (kTwo) {
+      if (two) load_tile2(wv2, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kPro == 1) {
+      float ss = 0.f;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+        if (kk < nkk) {
+          if (pro.res) nx[kk] = add_bf16x8(nx[kk], nr[kk]);
+          ss = rms_acc8(nx[kk], ss);
+        }
+      const float rs = rms_rsigma(ss, K, pro.eps);
+      if (prow < M && l32 == 0) rs_lds[prow] = rs;
+      __syncthreads();
+      finish_rs();
+      if (write_x && prow < M) {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+          if (kk < nkk)
+            st16(pro.xout + int64_t(prow) * pro.xo0 + (32 * kk + l32) * 8, nx[kk]);
+      }
+    }
 #pragma unroll
     for (int j = 0; j < R; ++j)
 #pragma unroll
-      for (int nt = 0; nt < kNT; ++nt) wv[j][nt] = ld16(wp[nt] + k + 32 * j);
-    batch(steps, wv, k);
+      for (int mt = 0; mt < kMT; ++mt) step(acc, wv[j], operand(av[mt][j], nv[j], mt), mt);
+    if constexpr (kTwo) {
+      if (two) {
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+#pragma unroll
+          for (int mt = 0; mt < kMT; ++mt)
+            step2(wv2[j], operand(av[mt][j], nv[j], mt), mt);
+      }
+    }
   };
-  using S4 = std::integral_constant<int, 4>;
-  if (nfull > 0) batch(S4{}, w_first, 0);
-  for (int b = 1; b < nfull; ++b) load_batch(S4{}, 128 * b);
-  const int kt = 128 * nfull;
-  if (rem == 1) load_batch(std::integral_constant<int, 1>{}, kt);
-  else if (rem == 2) load_batch(std::integral_constant<int, 2>{}, kt);
-  else if (rem == 3) load_batch(std::integral_constant<int, 3>{}, kt);
+  constexpr bool kOnce = kMT <= 2 && kNW <= 8;   // registers
+  const bool fits = kPro != 1 || (K <= 1024 && M <= kOnceRows && rem == 0);
+  if (kOnce && fits && nfull == 1) {
+    if (rem == 0) once(std::integral_constant<int, 4>{});
+    if constexpr (kPro != 1) {
+      if (rem == 1) once(std::integral_constant<int, 5>{});
+      else if (rem == 2) once(std::integral_constant<int, 6>{});
+      else if (rem == 3) once(std::integral_constant<int, 7>{});
+    }
+  } else {
+    if constexpr (kPro == 1) {
+      // rsigma of every row: 32 lanes per row, lane l summing the 8-element
+      // chunks (32 kk + l) * 8 in order, then the xor tree (rms_rsigma)
+      const int l32 = threadIdx.x & 31;
+      for (int row = threadIdx.x >> 5; row < M; row += 2 * kNW) {
+        const bf16_t *hr = x + int64_t(row) * xs0;
+        const bf16_t *rr = pro.res ? pro.res + int64_t(row) * pro.res0 : nullptr;
+        float ss = 0.f;
+        for (int kk = 0; kk < K / 256; ++kk) {
+          const int c = (32 * kk + l32) * 8;
+          u32x4_t t = ld16(hr + c);
+          if (rr) t = add_bf16x8(t, ld16(rr + c));
+          if (write_x) st16(pro.xout + int64_t(row) * pro.xo0 + c, t);
+          ss = rms_acc8(t, ss);
+        }
+        const float rs = rms_rsigma(ss, K, pro.eps);
+        if (l32 == 0) rs_lds[row] = rs;
+      }
+      __syncthreads();
+      finish_rs();
+    }
+    // all loads of a batch are issued before its first MFMA
+    auto load_batch = [&](auto steps, int k) {
+      constexpr int R = decltype(steps)::value;
+      u32x4_t wv[R][kNT], av[kMT][R], wv2[kTwo ? R : 1];
+#pragma unroll
+      for (int j = 0; j < R; ++j)
+#pragma unroll
+        for (int nt = 0; nt < kNT; ++nt) wv[j][nt] = ld16(wp[nt] + k + 32 * j);
+      if constexpr (kTwo) {
+        if (two) load_tile2(wv2, k);
+      }
+#pragma unroll
+      for (int mt = 0; mt < kMT; ++mt)
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+          u32x4_t nw8 = {0u, 0u, 0u, 0u};
+          if constexpr (kPro == 1) nw8 = ld16(nwp + k + 32 * j);
+          av[mt][j] = operand(load_raw(mt, k + 32 * j), nw8, mt);
+        }
+#pragma unroll
+      for (int j = 0; j < R; ++j)
+#pragma unroll
+        for (int mt = 0; mt < kMT; ++mt) step(acc, wv[j], av[mt][j], mt);
+      if constexpr (kTwo) {
+        if (two) {
+#pragma unroll
+          for (int j = 0; j < R; ++j)
+#pragma unroll
+            for (int mt = 0; mt < kMT; ++mt) step2(wv2[j], av[mt][j], mt);
+        }
+      }
+    };
+    for (int b = 0; b < nfull; ++b) load_batch(std::integral_constant<int, 4>{}, 128 * b);
+    const int kt = 128 * nfull;
+    if (rem == 1) load_batch(std::integral_constant<int, 1>{}, kt);
+    else if (rem == 2) load_batch(std::integral_constant<int, 2>{}, kt);
+    else if (rem == 3) load_batch(std::integral_constant<int, 3>{}, kt);
+  }
 
   // lane l of tile (mt, nt) holds rows mt*16 + 4(l/16) + i (i = 0..3) of
   // column 16 nt + l%16
@@ -317,6 +447,23 @@ __global__ __launch_bounds__(64 * kNW) void gemm_skinny_kernel(
         __hip_atomic_store(part + blockIdx.y * part_stride + int64_t(row) * N + n0 + cc, s,
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+  }
+  if constexpr (kTwo) {
+    if (two) {
+      __syncthreads();
+#pragma unroll
+      for (int mt = 0; mt < kMT; ++mt) red[wave][mt][lane] = acc2[mt];
+      __syncthreads();
+      for (int e = threadIdx.x; e < M * 16; e += 64 * kNW) {
+        const int row = e >> 4, cc = e & 15;
+        const int mt = row >> 4, src = cc + 16 * ((row & 15) >> 2);
+        float sum = 0.f;
+#pragma unroll
+        for (int wv = 0; wv < kNW; ++wv) sum += red[wv][mt][src][row & 3];
+        if (n2 + cc < N) y[int64_t(row) * ys0 + n2 + cc] = bf16_t(f32_to_bf16_bits(sum));
+      }
+    }
+    return;
   }
   if (n_split == 1) return;
   // The partial stores have completed before the count (a workgroup-scope
@@ -891,14 +1038,22 @@ struct SkinnyArgs {
   float *part;
   int32_t *cnt;
   ProArgs pro;
+  int over = 0;   // 16-column tiles that the first workgroups take besides their own
 };
 
 template <int kNW, int kMT, int kNT, int kPro, int kEpi = 0>
 void launch_skinny(const SkinnyArgs &a, hipStream_t st) {
   const int cols = 16 * (kEpi == 1 ? 1 : kNT);
-  const dim3 grid(unsigned((a.N + cols - 1) / cols), unsigned(a.split));
+  const dim3 grid(unsigned((a.N - 16 * a.over + cols - 1) / cols), unsigned(a.split));
+  if constexpr (kNW == 8 && kNT == 2 && kPro == 0 && kEpi == 0) {
+    if (a.over > 0) {
+      gemm_skinny_kernel<kNW, kMT, kNT, kPro, kEpi, true><<<grid, 64 * kNW, 0, st>>>(
+          a.x, a.xs0, a.w, a.ws0, a.y, a.ys0, a.M, a.N, a.K, a.part, a.cnt, a.pro, a.over);
+      return;
+    }
+  }
   gemm_skinny_kernel<kNW, kMT, kNT, kPro, kEpi><<<grid, 64 * kNW, 0, st>>>(
-      a.x, a.xs0, a.w, a.ws0, a.y, a.ys0, a.M, a.N, a.K, a.part, a.cnt, a.pro);
+      a.x, a.xs0, a.w, a.ws0, a.y, a.ys0, a.M, a.N, a.K, a.part, a.cnt, a.pro, 0);
 }
 
 template <int kNW, int kNT, int kPro, int kEpi = 0>
@@ -935,6 +1090,7 @@ void launch_skinny_plan(const SkinnyArgs &a, int nt, int nw, hipStream_t st) {
 // splits across workgroups, waves per workgroup.
 struct SkinnyPlan {
   int nt, blocks, split, nw;
+  int over;   // 16-column tiles past whole rounds of the CUs, left to the first workgroups
 };
 // Waves per workgroup for `groups` workgroups that each cover `ks` of K: grow
 // from 4 while the grid holds fewer than 2048 waves, each wave keeps at least
@@ -965,6 +1121,15 @@ SkinnyPlan skinny_plan(int N, int K, bool gate_up_pairs = false) {
   // Waves: enough workgroups x waves to keep the CUs streaming, each wave at
   // least one 128-wide batch of k.
   p.nw = skinny_waves(p.blocks * p.split, K / p.split);
+  // One or two blocks past whole rounds of the CUs (the GDN in_proj's 8224 =
+  // 256 x 32 + 32) go to the first workgroups, a tile each; more of them fill a
+  // round well enough.  Only where a wave reads its K slice in one batch
+  // (K / nw = 128), so that the tile's rows are requested with the others.
+  const int past = p.blocks % 256;
+  p.over = !gate_up_pairs && p.nt == 2 && p.nw == 8 && p.split == 1 && K == 128 * p.nw &&
+                   p.blocks > 256 && past >= 1 && past <= 2
+               ? (N - (p.blocks - past) * 32 + 15) / 16
+               : 0;
   return p;
 }
 
@@ -996,6 +1161,8 @@ static int run_skinny(SkinnyArgs a, int pro, void *workspace, int64_t workspace_
   } else if (p.split > 1) {  // no workspace: one workgroup per column block
     p.split = 1;
     p.nw = skinny_waves(p.blocks, a.K);
+  } else if (pro == 0) {
+    a.over = p.over;
   }
   if (pro == 1) launch_skinny_plan<1>(a, p.nt, p.nw, st);
   else if (pro == 2) launch_skinny_plan<2>(a, p.nt, p.nw, st);
@@ -1089,6 +1256,24 @@ extern "C" int64_t wy_gemm_2d_gate_up_swiglu_workspace_bytes(int M, int N, int K
   return kSplitPartOffset + int64_t(p.split) * M * 2 * N * 4;
 }
 
+// Gate/up pairs on the skinny kernel.
+static int run_gate_up(SkinnyArgs a, void *workspace, int64_t workspace_bytes, hipStream_t st) {
+  SkinnyPlan p = skinny_plan(a.N, a.K, true);
+  const int64_t need = wy_gemm_2d_gate_up_swiglu_workspace_bytes(a.M, a.N, a.K);
+  if (p.split > 1 && need > 0 && workspace_bytes >= need) {
+    a.split = p.split;
+    a.cnt = static_cast<int32_t *>(workspace);
+    a.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + kSplitPartOffset);
+  } else if (p.split > 1) {
+    p.split = 1;
+    p.nw = skinny_waves(p.blocks, a.K);
+  }
+  if (p.nw == 4) launch_skinny_m<4, 2, 0, 1>(a, st);
+  else if (p.nw == 8) launch_skinny_m<8, 2, 0, 1>(a, st);
+  else launch_skinny_m<16, 2, 0, 1>(a, st);
+  return wyh::launch_status();
+}
+
 extern "C" int wy_gemm_2d_gate_up_swiglu(const void *x, int64_t x_stride0, const void *w,
                                          int64_t w_stride0, void *y, int64_t y_stride0, int M,
                                          int N, int K, void *workspace, int64_t workspace_bytes,
@@ -1111,22 +1296,8 @@ extern "C" int wy_gemm_2d_gate_up_swiglu(const void *x, int64_t x_stride0, const
         static_cast<const bf16_t *>(x), x_stride0, static_cast<const bf16_t *>(w), w_stride0,
         static_cast<bf16_t *>(y), y_stride0, M, N, K, static_cast<hipStream_t>(stream));
   }
-  SkinnyArgs a{static_cast<const bf16_t *>(x), x_stride0, static_cast<const bf16_t *>(w),
-               w_stride0, static_cast<bf16_t *>(y), y_stride0, M, N, K, 1, nullptr, nullptr,
-               ProArgs{}};
-  SkinnyPlan p = skinny_plan(N, K, true);
-  const int64_t need = wy_gemm_2d_gate_up_swiglu_workspace_bytes(M, N, K);
-  if (p.split > 1 && need > 0 && workspace_bytes >= need) {
-    a.split = p.split;
-    a.cnt = static_cast<int32_t *>(workspace);
-    a.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + kSplitPartOffset);
-  } else if (p.split > 1) {
-    p.split = 1;
-    p.nw = skinny_waves(p.blocks, K);
-  }
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  if (p.nw == 4) launch_skinny_m<4, 2, 0, 1>(a, st);
-  else if (p.nw == 8) launch_skinny_m<8, 2, 0, 1>(a, st);
-  else launch_skinny_m<16, 2, 0, 1>(a, st);
-  return wyh::launch_status();
+  return run_gate_up({static_cast<const bf16_t *>(x), x_stride0,
+                      static_cast<const bf16_t *>(w), w_stride0, static_cast<bf16_t *>(y),
+                      y_stride0, M, N, K, 1, nullptr, nullptr, ProArgs{}},
+                     workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }

@@ -271,3 +271,20 @@ def test_fused_prologue_gemms_accept_unaligned_row_views(pkg, dev):
     y2 = pkg.swiglu_gemm_2d(gu, w)
     assert torch.equal(y2, pkg.gemm_2d(pkg.swiglu(gu[:, :1024].contiguous(),
                                                   gu[:, 1024:].contiguous()), w))
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("N", [8192, 8193, 8224, 8230, 8256, 8257])
+def test_gemm_2d_blocks_past_a_round(pkg, dev, M, N):
+    """The columns of one or two blocks past 256 of them go to the first workgroups
+    (N 8193 .. 8256); the columns are summed in the same order in
+    every form, so they equal the GEMM of the last rows of the weight alone."""
+    say(f"gemm_2d blocks past a round M={M} N={N}")
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn(M, 1024, generator=g).bfloat16()
+    w = (torch.randn(N, 1024, generator=g) * 0.05).bfloat16()
+    xd, wd = x.to(dev), w.to(dev)
+    y = pkg.gemm_2d(xd, wd)
+    check(y, x, w)
+    tail = pkg.gemm_2d(xd, wd[N - 4096:].contiguous())   # 128 blocks, no second ones
+    assert torch.equal(y[:, N - 4096:], tail)
