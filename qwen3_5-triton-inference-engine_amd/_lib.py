@@ -15,8 +15,8 @@ import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libwy_attn.so"
 
-_c_i64p = ctypes.POINTER(ctypes.c_int64)
 _vp = ctypes.c_void_p
+_c_i64p = _vp   # int64 arrays cross as addresses (strides()), ctypes arrays are taken too
 _i = ctypes.c_int
 _i64 = ctypes.c_int64
 _f = ctypes.c_float
@@ -142,15 +142,31 @@ def load() -> ctypes.CDLL:
     return lib
 
 
-def strides(t):
-    if t is None:
-        return None
-    s = t.stride()
-    return (ctypes.c_int64 * len(s))(*s)
+# The host side of a call is most of what a small one costs, so what every call
+# needs is kept at hand: the stride tuples met so far as int64 arrays with their
+# addresses (read-only to the library, and by value: a tuple of numbers, not a
+# tensor, is the key), and the bound functions.  Both only grow, to at most
+# _MAX_STRIDES entries (a few dozen bytes each) and one per entry point.
+_STRIDES: dict = {}
+_MAX_STRIDES = 4096
+_FNS: dict = {}
 
 
 def i64_array(values):
-    return (ctypes.c_int64 * len(values))(*values)
+    """The values as an int64 array for the library."""
+    key = tuple(values)
+    hit = _STRIDES.get(key)
+    if hit is not None:
+        return hit[1]
+    arr = (ctypes.c_int64 * len(key))(*key)
+    if len(_STRIDES) >= _MAX_STRIDES:
+        return arr   # lives as long as the caller's argument list
+    # of two threads that meet a tuple at once, both use the entry that is kept
+    return _STRIDES.setdefault(key, (arr, ctypes.addressof(arr)))[1]
+
+
+def strides(t):
+    return None if t is None else i64_array(t.stride())
 
 
 def ptr(t):
@@ -158,14 +174,20 @@ def ptr(t):
 
 
 def stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The raw handle of torch's current stream (the value of
+    ``torch.cuda.current_stream(device).cuda_stream``, without the object)."""
+    idx = device.index
+    return torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if idx is None else idx)
 
 
 def call(name: str, *args) -> None:
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    fn = _FNS.get(name)
+    if fn is None:
+        fn = _FNS.setdefault(name, getattr(load(), name))
+    rc = fn(*args)
     if rc != 0:
-        msg = lib.wy_status_string(rc).decode()
+        msg = load().wy_status_string(rc).decode()
         raise RuntimeError(f"{name} failed with code {rc}: {msg}")
 
 
@@ -178,10 +200,12 @@ _WORKSPACES: dict = {}
 
 
 def stream_workspace(device, tag: str, nbytes: int) -> torch.Tensor:
-    dev = torch.device(device)
+    dev = device if isinstance(device, torch.device) else torch.device(device)
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
-    key = (idx, stream(dev), tag)
-    bufs = _WORKSPACES.setdefault(key, [])
+    key = (idx, torch._C._cuda_getCurrentRawStream(idx), tag)
+    bufs = _WORKSPACES.get(key)
+    if bufs is None:
+        bufs = _WORKSPACES.setdefault(key, [])
     if not bufs or bufs[-1].numel() < nbytes:
         size = max(nbytes, 2 * bufs[-1].numel()) if bufs else nbytes
         bufs.append(torch.zeros(size, dtype=torch.uint8, device=dev))

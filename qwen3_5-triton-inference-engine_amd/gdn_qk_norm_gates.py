@@ -39,7 +39,7 @@ def gdn_qk_norm_gates(
     assert num_heads & (num_heads - 1) == 0
     assert head_dim & (head_dim - 1) == 0
     a_log, dt_bias = a_log.contiguous(), dt_bias.contiguous()
-    q_norm = torch.empty((token_num, num_heads, head_dim), dtype=q.dtype, device=q.device)
+    q_norm = q.new_empty((token_num, num_heads, head_dim))
     k_norm = torch.empty_like(q_norm)
     beta = torch.empty((token_num, num_heads), dtype=torch.float32, device=q.device)
     g = torch.empty_like(beta)

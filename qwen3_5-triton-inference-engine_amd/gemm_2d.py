@@ -29,7 +29,7 @@ def gemm_2d(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         x = x.contiguous()
     if weight.stride(1) != 1 or weight.stride(0) % 8 or weight.data_ptr() % 16:
         weight = weight.contiguous()
-    out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    out = x.new_empty((M, N))
     # Decode shapes with few column blocks split K across workgroups; the
     # split counters and fp32 partials live in a per-stream workspace.
     ws_bytes = _lib.load().wy_gemm_2d_workspace_bytes(M, N, K)
@@ -138,7 +138,7 @@ def gate_up_swiglu(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         gu = gemm_2d(x, weight)
         return swiglu(gu[:, :N], gu[:, N:])
     x = _rows16(x)
-    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    y = x.new_empty((M, N))
     ws_bytes = _lib.load().wy_gemm_2d_gate_up_swiglu_workspace_bytes(M, N, K)
     ws = _lib.stream_workspace(x.device, "gemm_split", ws_bytes) if ws_bytes > 0 else None
     _lib.call("wy_gemm_2d_gate_up_swiglu", _lib.ptr(x), x.stride(0), _lib.ptr(weight),
