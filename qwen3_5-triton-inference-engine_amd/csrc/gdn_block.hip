@@ -19,13 +19,28 @@ namespace {
 
 // acc = x[t-3] w0 + x[t-2] w1 + x[t-1] w2 + x[t] w3 (fp32, in tap order),
 // y = acc * sigmoid(acc) rounded to bf16.
-__device__ __forceinline__ float conv4_silu_f(float s1, float s2, float s3, float x, float w0,
-                                              float w1, float w2, float w3) {
+__device__ __forceinline__ float conv4_acc(float s1, float s2, float s3, float x, float w0,
+                                           float w1, float w2, float w3) {
   float acc = s1 * w0;
   acc = __fmaf_rn(s2, w1, acc);
   acc = __fmaf_rn(s3, w2, acc);
-  acc = __fmaf_rn(x, w3, acc);
+  return __fmaf_rn(x, w3, acc);
+}
+__device__ __forceinline__ float conv4_silu_f(float s1, float s2, float s3, float x, float w0,
+                                              float w1, float w2, float w3) {
+  const float acc = conv4_acc(s1, s2, s3, x, w0, w1, w2, w3);
   return acc * (1.0f / (1.0f + __expf(-acc)));
+}
+// The bits of the division 1 / d for 1 <= d <= 2^126 (and NaN for NaN): one
+// Newton step on v_rcp_f32, compared with the division for every such float.
+__device__ __forceinline__ float recip_ranged(float d) {
+  const float r = __builtin_amdgcn_rcpf(d);
+  return __fmaf_rn(__fmaf_rn(-d, r, 1.0f), r, r);
+}
+// acc * sigmoid(acc) as conv4_silu_f for acc >= kSiluLeast (1 + exp(87) < 2^126).
+constexpr float kSiluLeast = -87.0f;
+__device__ __forceinline__ float silu_ranged(float acc) {
+  return acc * recip_ranged(1.0f + __expf(-acc));
 }
 __device__ __forceinline__ uint32_t conv4_silu(float s1, float s2, float s3, float x, float w0,
                                                float w1, float w2, float w3) {
@@ -145,6 +160,7 @@ __global__ __launch_bounds__(128) void gdn_gated_rmsnorm_kernel(
 // arithmetic as the decode step (conv4_silu), so prefill and decode agree bit
 // for bit on the same window.
 constexpr int kConvRun = 16;
+constexpr int kConvVecRun = 4;  // the vectorised kernel's, measured there
 // Row counts from which the norm ops take the row-vectorised kernels (the
 // decode sizes keep one block per row, the same reduction either way).
 constexpr int kVecRows = 256;
@@ -187,16 +203,27 @@ __global__ __launch_bounds__(256) void conv4_prefill_kernel(
 // are lanes l ^ 4 / 2 / 1, offsets 4 / 2 / 1 are registers j ^ 4 / 2 / 1, the
 // halves are lanes l ^ 8.  fp addition is commutative, so every partial sum
 // is bit-identical to sum128's and the results match the one-thread-per-
-// element kernels (and the fused decode block) bit for bit.
+// element kernels (and the fused decode block) bit for bit.  The lane
+// exchanges are DPP moves inside the 16-lane row (l ^ 4 is the mirror of each
+// 8 lanes after the mirror of each 4): as LDS permutes, 25 a row, they kept
+// the LDS pipe busy for longer than the rows took from memory.
+template <int kCtrl>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xf, 0xf, false));
+}
 __device__ __forceinline__ float row_sum128(float (&v)[8]) {
+  constexpr int kQuadMirror = 0x1b, kQuadXor2 = 0x4e, kQuadXor1 = 0xb1, kHalfMirror = 0x141;
 #pragma unroll
-  for (int o = 4; o > 0; o >>= 1)
+  for (int j = 0; j < 8; ++j) v[j] += dpp<kHalfMirror>(dpp<kQuadMirror>(v[j]));
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] += __shfl_xor(v[j], o);
+  for (int j = 0; j < 8; ++j) v[j] += dpp<kQuadXor2>(v[j]);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] += dpp<kQuadXor1>(v[j]);
   const float a0 = v[0] + v[4], a1 = v[1] + v[5], a2 = v[2] + v[6], a3 = v[3] + v[7];
   const float b0 = a0 + a2, b1 = a1 + a3;
   const float h = b0 + b1;
-  return h + __shfl_xor(h, 8);
+  return h + row_ror<8>(h);
 }
 
 __device__ __forceinline__ void unpack8(const u32x4_t x, float (&f)[8]) {
@@ -207,35 +234,52 @@ __device__ __forceinline__ void unpack8(const u32x4_t x, float (&f)[8]) {
   }
 }
 
-// q/k norms and gates: 16 rows per 256-thread block, rows 2i (q) and 2i + 1
-// (k) of (token, head) pair 8 blockIdx + i.
+// q/k norms and gates: 32 (token, head) pairs per 256-thread block, each
+// 16-lane group the q and k rows of two of them (four 16-byte loads in flight
+// a lane); the gates of all 32 by the block's first 32 threads, not by one
+// lane of every fourth row.  Bound by memory, a copy's time: 16 heads x 4096
+// tokens 20.5 -> 12.3 us, 23772 tokens 104 -> 71 (5.5 TB/s).
+constexpr int kNormPairs = 32;
 __global__ __launch_bounds__(256) void gdn_qk_norm_gates_vec_kernel(const QkNormArgs p,
                                                                     int pairs) {
   const int grp = threadIdx.x >> 4, l = threadIdx.x & 15;
-  const int th = blockIdx.x * 8 + (grp >> 1);
-  const bool is_k = grp & 1;
-  if (th >= pairs) return;   // uniform over the 16-lane group
-  const int t = th / p.heads, h = th - t * p.heads;
-  const u32x4_t raw = ld16(is_k ? p.k + t * p.k_t + h * p.k_h + 8 * l
-                                : p.q + t * p.q_t + h * p.q_h + 8 * l);
-  float x[8], sq[8];
-  unpack8(raw, x);
+  const int base = blockIdx.x * kNormPairs;
+  u32x4_t raw[2][2];
+  int64_t to[2];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) sq[j] = x[j] * x[j];
-  const float r = rsqrtf(row_sum128(sq) + 1e-6f);
-  u32x4_t o;
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    o[e] = is_k ? (f32_to_bf16_bits(x[2 * e] * r) | (f32_to_bf16_bits(x[2 * e + 1] * r) << 16))
-                : (f32_to_bf16_bits((x[2 * e] * r) * p.q_scale) |
-                   (f32_to_bf16_bits((x[2 * e + 1] * r) * p.q_scale) << 16));
-  st16(is_k ? p.kn + t * p.kn_t + h * p.kn_h + 8 * l : p.qn + t * p.qn_t + h * p.qn_h + 8 * l, o);
-  if (!is_k && l == 0) {
+  for (int i = 0; i < 2; ++i) {
+    const unsigned th = unsigned(min(base + grp + 16 * i, pairs - 1));
+    const unsigned t = th / unsigned(p.heads), h = th - t * unsigned(p.heads);
+    raw[i][0] = ld16(p.q + t * p.q_t + h * p.q_h + 8 * l);
+    raw[i][1] = ld16(p.k + t * p.k_t + h * p.k_h + 8 * l);
+    to[i] = int64_t(th) * kDK + 8 * l;  // qn and kn are contiguous rows
+  }
+  if (int(threadIdx.x) < kNormPairs && base + int(threadIdx.x) < pairs) {
+    const unsigned th = unsigned(base) + threadIdx.x;
+    const unsigned t = th / unsigned(p.heads), h = th - t * unsigned(p.heads);
     float beta, g;
     gdn_gates(bf16_to_f32(p.a[t * p.a_t + h * p.a_h]), bf16_to_f32(p.b[t * p.b_t + h * p.b_h]),
               p.a_log[h], bf16_to_f32(p.dt_bias[h]), beta, g);
     p.beta[th] = beta;
     p.g[th] = g;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    if (base + grp + 16 * i >= pairs) break;  // uniform over the 16-lane group
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float x[8], sq[8];
+      unpack8(raw[i][u], x);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sq[j] = x[j] * x[j];
+      const float r = rsqrtf(row_sum128(sq) + 1e-6f);
+      u32x4_t o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        o[e] = u ? pack_bf16x2(x[2 * e] * r, x[2 * e + 1] * r)
+                 : pack_bf16x2((x[2 * e] * r) * p.q_scale, (x[2 * e + 1] * r) * p.q_scale);
+      st16((u ? p.kn : p.qn) + to[i], o);
+    }
   }
 }
 
@@ -268,29 +312,57 @@ __global__ __launch_bounds__(256) void gdn_gated_rmsnorm_vec_kernel(
 
 // conv4 prefill with 8 consecutive channels per thread (16-byte loads and
 // stores); per channel the same window and arithmetic as conv4_prefill_kernel.
+//
+// Bound by memory, 24 KB a token of 6144 channels, if the VALU work (13
+// instructions an element, two of them transcendental) stays beside it: the
+// weights come as whole 16-byte rows ahead of the window rows and nothing in
+// the body waits for a later load, so a wave computes on its first rows while
+// the last ones land; runs of 4 tokens leave enough waves for one to load
+// while another computes.  A run's first 3 rows are another run's last:
+// workgroup b is on XCD b % 8, so each XCD takes a consecutive range of runs
+// and finds them in its L2.  6144 channels, us by run length, without / with
+// that mapping: 4096 tokens 4: 26.5 / 21.1, 8: 24.6 / 22.1, 16: 25.4 / 24.8;
+// 23772 tokens 130 / 120, 140 / 120, 136 / 126.  With 2-byte weight loads, the
+// library division and runs of 16 it took 29.3 and 137; a copy takes 15 and 108.
+template <int kRun, bool kRowsW, bool kSeq>
 __global__ __launch_bounds__(256) void conv4_prefill_vec_kernel(
     const bf16_t *__restrict__ x, int64_t x_t, const bf16_t *__restrict__ w, int64_t w_c,
     int64_t w_k, bf16_t *__restrict__ out, int64_t o_t, const int32_t *__restrict__ seq_start,
-    int T, int C) {
-  const int c0 = (blockIdx.x * 256 + threadIdx.x) * 8;
-  const int t0 = blockIdx.y * kConvRun;
-  if (c0 >= C) return;
-  float wt[4][8];
+    int T, int C, int xb) {
+  const int tile = int(blockIdx.x & 7) * int(gridDim.x >> 3) + int(blockIdx.x >> 3);
+  const int run = tile / xb;
+  const int c0 = ((tile - run * xb) * 256 + threadIdx.x) * 8;
+  const int t0 = run * kRun;
+  if (c0 >= C || t0 >= T) return;
+  u32x4_t wr[4];
+  if constexpr (kRowsW) {
 #pragma unroll
-  for (int k = 0; k < 4; ++k)
+    for (int k = 0; k < 4; ++k) wr[k] = ld16(w + k * w_k + c0);
+  } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) wt[k][j] = bf16_to_f32(w[(c0 + j) * w_c + k * w_k]);
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        wr[k][e] = w[(c0 + 2 * e) * w_c + k * w_k] |
+                   (uint32_t(w[(c0 + 2 * e + 1) * w_c + k * w_k]) << 16);
+  }
+  int lo[kRun];
+#pragma unroll
+  for (int i = 0; i < kRun; ++i) lo[i] = kSeq ? seq_start[min(t0 + i, T - 1)] : 0;
   // win[j] = x[t0 - 3 + j, c0 .. c0 + 7].  Rows outside [0, T) read a clamped
   // row instead of branching round the load (loads that only some paths
   // issue make every later wait a wait for all of them): a row before 0 lies
   // before every sequence's start and is masked below, a row from T on only
   // feeds tokens from T on, which are not computed.
-  u32x4_t win[kConvRun + 3];
+  u32x4_t win[kRun + 3];
 #pragma unroll
-  for (int j = 0; j < kConvRun + 3; ++j) {
+  for (int j = 0; j < kRun + 3; ++j) {
     const int t = min(max(t0 - 3 + j, 0), T - 1);
     win[j] = ld16(x + int64_t(t) * x_t + c0);
   }
+  float wt[4][8];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) unpack8(wr[k], wt[k]);
   // each window row is unpacked once into a rolling 4-row float window; the
   // per-row masks for rows before the sequence's start are only evaluated for
   // a token whose window reaches past it (a block-uniform branch); the pair
@@ -300,7 +372,7 @@ __global__ __launch_bounds__(256) void conv4_prefill_vec_kernel(
   unpack8(win[1], f[1]);
   unpack8(win[2], f[2]);
 #pragma unroll
-  for (int i = 0; i < kConvRun; ++i) {
+  for (int i = 0; i < kRun; ++i) {
     const int t = t0 + i;
     if (t >= T) break;
     unpack8(win[i + 3], f[(i + 3) & 3]);
@@ -308,20 +380,17 @@ __global__ __launch_bounds__(256) void conv4_prefill_vec_kernel(
     const float(&a1)[8] = f[(i + 1) & 3];
     const float(&a2)[8] = f[(i + 2) & 3];
     const float(&a3)[8] = f[(i + 3) & 3];
-    const int lo = seq_start ? seq_start[t] : 0;
+    float acc[8], least = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      acc[j] = conv4_acc(a0[j], a1[j], a2[j], a3[j], wt[0][j], wt[1][j], wt[2][j], wt[3][j]);
+      least = fminf(least, acc[j]);
+    }
     u32x4_t o;
-    if (t - 3 >= lo) {
+    if (t - 3 >= lo[i] && __ballot(least < kSiluLeast) == 0) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float y[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int j = 2 * e + u;
-          y[u] = conv4_silu_f(a0[j], a1[j], a2[j], a3[j], wt[0][j], wt[1][j], wt[2][j],
-                              wt[3][j]);
-        }
-        o[e] = pack_bf16x2(y[0], y[1]);
-      }
+      for (int e = 0; e < 4; ++e)
+        o[e] = pack_bf16x2(silu_ranged(acc[2 * e]), silu_ranged(acc[2 * e + 1]));
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -329,8 +398,8 @@ __global__ __launch_bounds__(256) void conv4_prefill_vec_kernel(
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const int j = 2 * e + u;
-          y[u] = conv4_silu_f(t - 3 >= lo ? a0[j] : 0.f, t - 2 >= lo ? a1[j] : 0.f,
-                              t - 1 >= lo ? a2[j] : 0.f, a3[j], wt[0][j], wt[1][j], wt[2][j],
+          y[u] = conv4_silu_f(t - 3 >= lo[i] ? a0[j] : 0.f, t - 2 >= lo[i] ? a1[j] : 0.f,
+                              t - 1 >= lo[i] ? a2[j] : 0.f, a3[j], wt[0][j], wt[1][j], wt[2][j],
                               wt[3][j]);
         }
         o[e] = pack_bf16x2(y[0], y[1]);
@@ -538,7 +607,7 @@ extern "C" int wy_gdn_qk_norm_gates(const void *q, const int64_t *q_strides, con
                    wyh::aligned16(q) && wyh::aligned16(k) && wyh::aligned16(q_norm) &&
                    wyh::aligned16(k_norm);
   if (vec && pairs >= kVecRows)
-    gdn_qk_norm_gates_vec_kernel<<<unsigned((pairs + 7) / 8), 256, 0,
+    gdn_qk_norm_gates_vec_kernel<<<unsigned((pairs + kNormPairs - 1) / kNormPairs), 256, 0,
                                    static_cast<hipStream_t>(stream)>>>(p, pairs);
   else
     gdn_qk_norm_gates_kernel<<<unsigned(pairs), 256, 0, static_cast<hipStream_t>(stream)>>>(p);
@@ -623,11 +692,19 @@ extern "C" int wy_depthwise_causal_conv4_prefill(const void *x, const int64_t *x
   const unsigned runs = unsigned((tokens + kConvRun - 1) / kConvRun);
   if (x_strides[1] == 1 && out_strides[1] == 1 && channels % 8 == 0 &&
       ((x_strides[0] | out_strides[0]) & 7) == 0 && wyh::aligned16(x) && wyh::aligned16(out)) {
-    conv4_prefill_vec_kernel<<<dim3(unsigned((channels / 8 + 255) / 256), runs), 256, 0,
-                               static_cast<hipStream_t>(stream)>>>(
+    const bool w_rows = w_stride_c == 1 && w_stride_k % 8 == 0 && wyh::aligned16(weight);
+    const unsigned vruns = unsigned((tokens + kConvVecRun - 1) / kConvVecRun);
+    const int xb = (channels / 8 + 255) / 256;
+    auto *kernel =
+        w_rows ? (seq_start ? conv4_prefill_vec_kernel<kConvVecRun, true, true>
+                            : conv4_prefill_vec_kernel<kConvVecRun, true, false>)
+               : (seq_start ? conv4_prefill_vec_kernel<kConvVecRun, false, true>
+                            : conv4_prefill_vec_kernel<kConvVecRun, false, false>);
+    const unsigned tiles = unsigned(xb) * vruns;
+    kernel<<<(tiles + 7) / 8 * 8, 256, 0, static_cast<hipStream_t>(stream)>>>(
         static_cast<const bf16_t *>(x), x_strides[0], static_cast<const bf16_t *>(weight),
         w_stride_c, w_stride_k, static_cast<bf16_t *>(out), out_strides[0], seq_start, tokens,
-        channels);
+        channels, xb);
     return wyh::launch_status();
   }
   const dim3 grid(unsigned((channels + 255) / 256), runs);

@@ -216,3 +216,39 @@ def test_row_vectorised_norms_equal_per_row_kernels(pkg, dev):
     for i in range(4):
         assert torch.equal(big[i], torch.cat([r[i] for r in rows])), i
     assert torch.equal(nbig, torch.cat(nrows))
+
+
+@pytest.mark.parametrize("T, Cs", [(1, 8), (3, 8), (4, 640), (5, 2048), (31, 2056), (130, 6144)])
+def test_conv4_prefill_forms_same_bits(pkg, dev, T, Cs):
+    """Eight channels a thread (either weight layout, with and without sequence
+    starts, any starts) and one channel a thread (inputs whose channels are not
+    adjacent) give the same bits, also where the SiLU's exp leaves the range
+    of the short reciprocal."""
+    say(f"conv4 prefill forms T={T} C={Cs}")
+    gen = torch.Generator().manual_seed(T + Cs)
+    x = torch.randn(T, Cs, generator=gen)
+    x[T // 2] *= 60.0  # sums beyond +-87: the division itself
+    x = x.to(torch.bfloat16).to(dev)
+    w = torch.randn(Cs, 4, generator=gen).to(torch.bfloat16).to(dev)
+    w_rows = w.t().contiguous().t()  # channel stride 1
+    apart = torch.empty(T, Cs, 2, dtype=torch.bfloat16, device=dev)[..., 0]
+    apart.copy_(x)
+    starts = torch.randint(0, T, (T,), generator=gen, dtype=torch.int32).to(dev)
+    for s in (None, starts):
+        ref = pkg.depthwise_causal_conv4_prefill(apart, w, s)
+        for wt in (w, w_rows):
+            assert torch.equal(pkg.depthwise_causal_conv4_prefill(x, wt, s), ref)
+
+
+@pytest.mark.parametrize("rows", [255, 256, 257, 287, 289])
+def test_qk_norm_gates_last_block(pkg, dev, rows):
+    """One head, so rows are tokens: both sides of the row count that takes the
+    row-vectorised kernel, and blocks of 32 pairs that end ragged."""
+    say(f"qk norm gates rows={rows}")
+    gen = torch.Generator().manual_seed(rows)
+    q, k = (torch.randn(rows, 1, D, generator=gen).to(torch.bfloat16) for _ in range(2))
+    a, b = (torch.randn(rows, 1, generator=gen).to(torch.bfloat16) for _ in range(2))
+    a_log, dt = torch.rand(1, generator=gen), torch.randn(1, generator=gen).to(torch.bfloat16)
+    got = pkg.gdn_qk_norm_gates(*(t.to(dev) for t in (q, k, a, b, a_log, dt)))
+    for x, ref in zip(got, go.gdn_qk_norm_gates(q, k, a, b, a_log, dt)):
+        close(x, ref)
