@@ -140,10 +140,16 @@ __device__ __forceinline__ float sum16(float v) {
 
 // Raw buffer resource over one cache page (bounds check off: the launcher has
 // validated the strides, and every offset stays inside the page).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t page_rsrc(const bf16_t *base) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(base), 0, -1, 0x00020000);
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t page_rsrc(const bf16_t *base, int bytes = -1) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(base), 0, bytes, 0x00020000);
 }
 
+// The attention block's prologue inputs of one lane besides its row piece: the
+// piece of that row's norm weight, of the new V row, and rotary frequencies.
+struct ProInputs {
+  u32x4_t w, vn;
+  float fq, fq_new;
+};
 
 
 // ctx = bf16(A / L), then optionally bf16(ctx * sigmoid(gate)): the same two
@@ -432,7 +438,26 @@ void paged_decode_split_kernel(const DecodeArgs a) {
   const bf16_t *q_src = a.q + b * a.qs_b + (h * kG + r_q) * a.qs_h + c_q;
   const bool q_fast = threadIdx.x < kG * kD / 8 && (kProlog || a.qs_d == 1);
   u32x4_t q_pre = {0u, 0u, 0u, 0u};
-  if (q_fast) q_pre = ld16(q_src);
+  // The attention block's other inputs of the prologue (norm weights, rotary
+  // frequencies, the new token's raw rows) are requested here too, by every
+  // wave: all of them are then older than the page loads, which start before
+  // the prologue needs them.
+  ProInputs pi = {};
+  if constexpr (kProlog) {
+    const int half = a.rope_dim / 2, c = (lane & 31) * 8;
+    static_assert(kG * kD / 8 <= 64 * (kW - 1), "the last wave holds no query rows");
+    const bool lw = wave == kW - 1;
+    const bf16_t *q_row = a.q + b * a.qs_b + (h * kG + (r_q & (kG - 1))) * a.qs_h + c;
+    q_pre = ld16(lw ? a.kn + b * a.kn_b + h * a.kn_h + c : q_row);
+    pi.w = ld16((lw ? a.kw : a.qw) + c);
+    pi.vn = ld16(a.vn + b * a.vn_b + h * a.vn_h + c);
+    // without rotation (rope_dim 0) there may be no frequencies to read
+    const float *fq = half ? a.inv_freq : reinterpret_cast<const float *>(a.qw);
+    pi.fq = fq[half ? threadIdx.x % half : 0];
+    pi.fq_new = fq[half ? lane % half : 0];
+  } else if (q_fast) {
+    q_pre = ld16(q_src);
+  }
   // The block-table entry of this wave's first page is requested together
   // with the q rows (and, in the direct order, with pos: for the usual
   // partition, pps == min_pps, its index is known before pos), so the first
@@ -472,15 +497,6 @@ void paged_decode_split_kernel(const DecodeArgs a) {
   u32x2_t gate_pre = {0u, 0u};
   if (kFused && a.gate && wave < kG) gate_pre = load_gate4(a, b, h * kG + wave, lane * 4);
 
-  float m_run[kG], l_run[kG], acc[kG][4];
-#pragma unroll
-  for (int r = 0; r < kG; ++r) {
-    m_run[r] = -INFINITY;
-    l_run[r] = 0.f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc[r][e] = 0.f;
-  }
-
   const bf16_t *kh = a.kc + h * a.kc_h;
   const bf16_t *vh = a.vc + h * a.vc_h;
   const int last_page = (seq_len - 1) / kPage;
@@ -504,6 +520,17 @@ void paged_decode_split_kernel(const DecodeArgs a) {
   u32x4_t kr[8];
   u32x2_t vr[kPage];
   int64_t phys_next = 0;
+  int page_bytes = -1;
+  if constexpr (kProlog) {
+    // Read back into a scalar register by hand: left in a vector register, the
+    // resource turns every page load into a loop over lanes.  The s_nops are
+    // the wait states after the VALU write of the operand and before a
+    // buffer load that reads the result, which the compiler does not add
+    // round an asm.
+    asm volatile("s_nop 1\n\tv_readfirstlane_b32 %0, %1\n\ts_nop 4"
+                 : "=s"(page_bytes)
+                 : "v"(npw > 0 ? -1 : 0));
+  }
   // Page loads are buffer loads off a per-page resource: one lane-offset
   // register per operand and the row/column steps in the scalar offset.
   const uint32_t k_voff = uint32_t(n16 * a.kc_s + g4 * 8) * 2u;
@@ -512,18 +539,18 @@ void paged_decode_split_kernel(const DecodeArgs a) {
   auto issue_k = [&](int i) {
     phys_next = bt_ahead;
     if (i + 1 < npw) bt_ahead = bt_s[p0 + wave + (i + 1) * kW];
-    const __amdgpu_buffer_rsrc_t rk = page_rsrc(kh + phys_next * a.kc_p);
+    const __amdgpu_buffer_rsrc_t rk = page_rsrc(kh + phys_next * a.kc_p, page_bytes);
 #pragma unroll
     for (int e = 0; e < 8; ++e) kr[e] = __builtin_amdgcn_raw_buffer_load_b128(rk, k_voff, 64 * e, 0);
   };
   auto issue_v = [&](int i) {
-    const __amdgpu_buffer_rsrc_t rv = page_rsrc(vh + phys_next * a.vc_p);
+    const __amdgpu_buffer_rsrc_t rv = page_rsrc(vh + phys_next * a.vc_p, page_bytes);
 #pragma unroll
     for (int e = 0; e < kPage; ++e)
       vr[e] = __builtin_amdgcn_raw_buffer_load_b64(rv, v_voff, v_row_bytes * e, 0);
   };
   auto issue_v_pair = [&](int j) {  // rows 2j, 2j+1 of the next page
-    const __amdgpu_buffer_rsrc_t rv = page_rsrc(vh + phys_next * a.vc_p);
+    const __amdgpu_buffer_rsrc_t rv = page_rsrc(vh + phys_next * a.vc_p, page_bytes);
     vr[2 * j] = __builtin_amdgcn_raw_buffer_load_b64(rv, v_voff, v_row_bytes * (2 * j), 0);
     vr[2 * j + 1] = __builtin_amdgcn_raw_buffer_load_b64(rv, v_voff, v_row_bytes * (2 * j + 1), 0);
   };
@@ -543,21 +570,18 @@ void paged_decode_split_kernel(const DecodeArgs a) {
     u32x4_t krow = {0u, 0u, 0u, 0u};
     if constexpr (kProlog) {
       // RMSNorm + partial RoPE of the raw key row (both 32-lane halves compute it)
-      const u32x4_t xw = ld16(knrow + c);
-      const u32x4_t ww = ld16(a.kw + c);
+      const u32x4_t xw = q_pre;
+      const u32x4_t ww = pi.w;
       // chunk l (dims 8l..8l+7) pairs with chunk l +- half/8
       const int hc = a.rope_dim / 16, l32 = lane & 31;
       const bool first = l32 < hc, second = l32 >= hc && l32 < 2 * hc;
       const int partner = (lane & 32) | (first ? l32 + hc : second ? l32 - hc : l32);
       const float pf = float(seq_len - 1);  // = float(pos[b])
-      float sn8[8], cs8[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        sn8[e] = 0.f;
-        cs8[e] = 1.f;
-        if (first || second)
-          rope_sincos(pf, a.inv_freq[(first ? c : c - 8 * hc) + e], sn8[e], cs8[e]);
-      }
+      // lane j computes pair j's sine and cosine (at most 64 pairs), the lanes
+      // that rotate fetch their eight
+      float sn_j, cs_j;
+      rope_sincos(pf, pi.fq_new, sn_j, cs_j);
+      const int j0 = (first ? c : c - 8 * hc) & 63;
       const float rs = rms_rsigma(rms_acc8(xw, 0.f), kD, a.eps);
       float y[8];
 #pragma unroll
@@ -571,14 +595,15 @@ void paged_decode_split_kernel(const DecodeArgs a) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const float other = __shfl(y[e + u], partner);
+          const float sn = __shfl(sn_j, j0 + e + u), cs = __shfl(cs_j, j0 + e + u);
           o[u] = y[e + u];
           if (first || second) {
             float o1, o2;
             if (first) {
-              rope_rotate(y[e + u], other, cs8[e + u], sn8[e + u], o1, o2);
+              rope_rotate(y[e + u], other, cs, sn, o1, o2);
               o[u] = o1;
             } else {
-              rope_rotate(other, y[e + u], cs8[e + u], sn8[e + u], o1, o2);
+              rope_rotate(other, y[e + u], cs, sn, o1, o2);
               o[u] = o2;
             }
           }
@@ -586,32 +611,44 @@ void paged_decode_split_kernel(const DecodeArgs a) {
         krow[e / 2] = pack_bf16x2(o[0], o[1]);
       }
     }
-    const int64_t phys = btrow[last_page];
-    if (lane < 32) {
-      st16(&sm.kn[c], krow);
-      st16(a.kc + phys * a.kc_p + h * a.kc_h + last_slot * a.kc_s + c, krow);
-    } else {
-      const u32x4_t vrow = ld16(vnrow + c);
-      st16(&sm.vn[c], vrow);
-      st16(a.vc + phys * a.vc_p + h * a.vc_h + last_slot * a.vc_s + c, vrow);
-    }
+    // Scalar page and row addresses, made opaque: the lanes' choice between
+    // them must not become a vector load of either's parts, which would wait
+    // for every page load in flight.
+    const int64_t phys = bt_s[last_page];
+    typedef __attribute__((address_space(1))) bf16_t *global_t;
+    global_t krow_dst = (global_t)(a.kc + phys * a.kc_p + h * a.kc_h + last_slot * a.kc_s);
+    global_t vrow_dst = (global_t)(a.vc + phys * a.vc_p + h * a.vc_h + last_slot * a.vc_s);
+    asm volatile("" : "+s"(krow_dst), "+s"(vrow_dst));
+    const u32x4_t vrow = kProlog ? pi.vn : ld16(vnrow + c);
+    st16(lane < 32 ? &sm.kn[c] : &sm.vn[c], lane < 32 ? krow : vrow);
+    *(__attribute__((address_space(1))) u32x4_t *)((lane < 32 ? krow_dst : vrow_dst) + c) =
+        lane < 32 ? krow : vrow;
   };
 
   // The group's 4 query rows, staged once in LDS; each page rebuilds the MFMA
   // A operand from it (rows 4..15 of the operand are zero).
   if constexpr (kProlog) {
+    // The first page's K and V travel while the prologue runs (a wave without
+    // pages has an empty buffer: every wave issues the same loads, so the
+    // prologue waits for its own, older ones alone).  A small batch's launch is
+    // a chain of memory round trips: table entry, prologue inputs, page,
+    // merge.  With the second and third one behind the other, 3001 tokens of one
+    // sequence took 15.9 us a launch; together 14.1.  32 sequences of
+    // 128..2048 tokens: 22.7 -> 21.4.
+    issue_k(0);
+    issue_v(0);
     if (has_new && wave == kW - 1) stage_new();
     // The RoPE inputs are fetched with the rows: lane i later rotates pair
     // (head i / half, j = i % half).
     const int half = a.rope_dim / 2;
     const float pf = float(seq_len - 1);  // = float(pos[b])
     float sn = 0.f, cs = 1.f;
-    if (threadIdx.x < kG * half) rope_sincos(pf, a.inv_freq[threadIdx.x % half], sn, cs);
+    if (threadIdx.x < kG * half) rope_sincos(pf, pi.fq, sn, cs);
     // RMSNorm: 32 lanes per row, 8 elements each (rms_rsigma's layout).
     if (threadIdx.x < kG * kD / 8) {
       const int r = threadIdx.x >> 5, c = (threadIdx.x & 31) * 8;
       const u32x4_t xw = q_pre;  // q row r, dims c..c+7 (r == r_q, c == c_q)
-      const u32x4_t ww = ld16(a.qw + c);
+      const u32x4_t ww = pi.w;
       const float ss = rms_acc8(xw, 0.f);
       const float rs = rms_rsigma(ss, kD, a.eps);
       u32x4_t y;
@@ -648,6 +685,15 @@ void paged_decode_split_kernel(const DecodeArgs a) {
   __syncthreads();
 
   WY_DSTAMP(2);
+  float m_run[kG], l_run[kG], acc[kG][4];
+#pragma unroll
+  for (int r = 0; r < kG; ++r) {
+    m_run[r] = -INFINITY;
+    l_run[r] = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[r][e] = 0.f;
+  }
+
   f32x4_t sc_new = {0.f, 0.f, 0.f, 0.f};
   u32x2_t vnew = {0u, 0u};
   bool owns_new = false;
@@ -680,7 +726,7 @@ void paged_decode_split_kernel(const DecodeArgs a) {
     }
   }
 
-  if (npw > 0) {
+  if (!kProlog && npw > 0) {
     issue_k(0);
     issue_v(0);
   }

@@ -647,6 +647,31 @@ def test_decode_block_equals_op_sequence(pkg, dev):
     assert int(sc1.counters.abs().sum()) == 0
 
 
+@pytest.mark.parametrize("rotary", [16, 48, 112, 128])
+@pytest.mark.parametrize("lens", [[1, 16, 17, 65, 200], [40] * 10 + [3, 64, 500, 1, 33, 128, 129]],
+                         ids=["direct", "balanced"])
+def test_decode_block_rotary_widths(pkg, dev, lens, rotary):
+    """Pair counts that do and do not divide a wavefront, splits whose last
+    waves have no page, in both workgroup orders: the block, whose waves
+    request every input before the prologue, equals the op sequence."""
+    say(f"decode attention block rotary={rotary} B={len(lens)}")
+    c = _block_case(torch.Generator().manual_seed(rotary + len(lens)), lens)
+    B = c["B"]
+    inv = (10000.0 ** (-torch.arange(0, rotary, 2).float() / rotary)).to(dev)
+    fg, bt, pos = c["fused"].to(dev), c["bt"].to(dev), c["pos"].to(dev)
+    qw, kw = c["qw"].to(dev), c["kw"].to(dev)
+    kc1, vc1 = c["kc"].to(dev), c["vc"].to(dev)
+    kc2, vc2 = kc1.clone(), vc1.clone()
+    scs = [pkg.allocate_split_scratch(HQ, D, batch=B, device=dev) for _ in range(2)]
+    out1 = pkg.decode_attention_block(fg, qw, kw, 1e-6, inv, rotary, pos, kc1, vc1, bt, scs[0])
+    q = pkg.qwen_rmsnorm(fg[:, :2048].view(B, HQ, D), qw, 1e-6)
+    k = pkg.qwen_rmsnorm(fg[:, 4096:4608].view(B, HKV, D), kw, 1e-6)
+    out2 = pkg.decode_attention_step(q, k, fg[:, 4608:], fg[:, 2048:4096], inv, rotary, pos,
+                                     kc2, vc2, bt, scs[1])
+    assert torch.equal(kc1, kc2) and torch.equal(vc1, vc2)
+    assert torch.equal(out1, out2)
+
+
 def test_decode_block_vs_oracle(pkg, dev):
     """The block against the reference op sequence computed by the oracle."""
     say("decode attention block vs oracle")
