@@ -203,27 +203,17 @@ __global__ __launch_bounds__(256) void conv4_prefill_kernel(
 // are lanes l ^ 4 / 2 / 1, offsets 4 / 2 / 1 are registers j ^ 4 / 2 / 1, the
 // halves are lanes l ^ 8.  fp addition is commutative, so every partial sum
 // is bit-identical to sum128's and the results match the one-thread-per-
-// element kernels (and the fused decode block) bit for bit.  The lane
-// exchanges are DPP moves inside the 16-lane row (l ^ 4 is the mirror of each
-// 8 lanes after the mirror of each 4): as LDS permutes, 25 a row, they kept
-// the LDS pipe busy for longer than the rows took from memory.
-template <int kCtrl>
-__device__ __forceinline__ float dpp(float v) {
-  return __int_as_float(
-      __builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xf, 0xf, false));
-}
+// element kernels (and the fused decode block) bit for bit.  (As LDS permutes
+// the exchanges, 25 a row, kept the LDS pipe busy for longer than the rows took
+// from memory.)
 __device__ __forceinline__ float row_sum128(float (&v)[8]) {
-  constexpr int kQuadMirror = 0x1b, kQuadXor2 = 0x4e, kQuadXor1 = 0xb1, kHalfMirror = 0x141;
+  const auto add = [](float a, float b) { return a + b; };
 #pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] += dpp<kHalfMirror>(dpp<kQuadMirror>(v[j]));
-#pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] += dpp<kQuadXor2>(v[j]);
-#pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] += dpp<kQuadXor1>(v[j]);
+  for (int j = 0; j < 8; ++j) v[j] = xor_reduce<4>(v[j], add);
   const float a0 = v[0] + v[4], a1 = v[1] + v[5], a2 = v[2] + v[6], a3 = v[3] + v[7];
   const float b0 = a0 + a2, b1 = a1 + a3;
   const float h = b0 + b1;
-  return h + row_ror<8>(h);
+  return xor_step<8>(h, add);
 }
 
 __device__ __forceinline__ void unpack8(const u32x4_t x, float (&f)[8]) {

@@ -57,15 +57,44 @@ __device__ __forceinline__ void st16_nt(void *p, u32x4_t v) {
   __builtin_nontemporal_store(v, reinterpret_cast<u32x4_t *>(p));
 }
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
+// Butterfly reductions, offsets 32, 16, 8, 4, 2, 1: step<O> combines lane l with
+// lane l ^ O.  The exchanges are VALU moves (DPP inside a 16-lane row, row and
+// half swaps above it); as LDS permutes each step waited about 120 cycles on
+// the latency chains of the decode kernels.  Every lane a value comes from must
+// be active.
+template <int kCtrl>
+__device__ __forceinline__ float dpp_mov(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, 0xf, 0xf, false));
+}
+template <int kOff, typename Op>
+__device__ __forceinline__ float xor_step(float v, Op op) {
+  static_assert(kOff == 32 || kOff == 16 || kOff == 8 || kOff == 4 || kOff == 2 || kOff == 1);
+  if constexpr (kOff >= 16) {
+    // swapping a register with its copy leaves both halves' values in every lane
+    const uint32_t u = __float_as_uint(v);
+    const auto r = kOff == 32 ? __builtin_amdgcn_permlane32_swap(u, u, false, false)
+                              : __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  } else if constexpr (kOff == 8) {
+    return op(v, dpp_mov<0x128>(v));  // row_ror:8
+  } else if constexpr (kOff == 4) {
+    return op(v, dpp_mov<0x141>(dpp_mov<0x1b>(v)));  // mirror of 4, then of 8
+  } else {
+    return op(v, dpp_mov<kOff == 2 ? 0x4e : 0xb1>(v));  // quad_perm
+  }
+}
+template <int kFrom, typename Op>
+__device__ __forceinline__ float xor_reduce(float v, Op op) {
+  v = xor_step<kFrom>(v, op);
+  if constexpr (kFrom > 1) v = xor_reduce<kFrom / 2>(v, op);
   return v;
 }
+__device__ __forceinline__ float wave_max(float v) {
+  return xor_reduce<32>(v, [](float a, float b) { return fmaxf(a, b); });
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+  return xor_reduce<32>(v, [](float a, float b) { return a + b; });
 }
 
 // ---- shared by the standalone RMSNorm / RoPE kernels and the fused decode
@@ -115,9 +144,7 @@ __device__ __forceinline__ float rms_acc8(u32x4_t xw, float ss) {
   return ss;
 }
 __device__ __forceinline__ float rms_rsigma(float sumsq_lane, int d_model, float eps) {
-  float s = sumsq_lane;
-#pragma unroll
-  for (int o = 16; o > 0; o >>= 1) s += __shfl_xor(s, o);
+  const float s = xor_reduce<16>(sumsq_lane, [](float a, float b) { return a + b; });
   return rsqrtf(s / float(d_model) + eps);
 }
 __device__ __forceinline__ float rms_apply(float x, float rsigma, float w) {
