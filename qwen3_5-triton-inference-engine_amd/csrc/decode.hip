@@ -540,7 +540,7 @@ void paged_decode_split_kernel(const DecodeArgs a) {
     // buffer load that reads the result, which the compiler does not add
     // round an asm.
     asm volatile("s_nop 1\n\tv_readfirstlane_b32 %0, %1\n\ts_nop 4"
-                 : "=s"(page_bytes)
+                 : "=&s"(page_bytes)
                  : "v"(npw > 0 ? -1 : 0));
   }
   // Page loads are buffer loads off a per-page resource: one lane-offset
