@@ -8,8 +8,8 @@ layer (8 q / 2 kv heads of 256, partial RoPE on 64 dims, theta 1e7), the
 others Gated DeltaNet layers (16 heads of 128), hidden 1024, MLP 3584, a tied
 248320 x 1024 embedding / LM head.  Per layer a decode step runs
 
-    rmsnorm -> fused projection GEMV -> mixer block (one launch) -> out GEMV
-    -> residual add -> rmsnorm -> gate_up GEMV -> SwiGLU -> down GEMV -> residual add
+    residual add + rmsnorm -> fused projection GEMV -> mixer block (one launch)
+    -> out GEMV -> residual add + rmsnorm -> gate_up GEMV + SwiGLU -> down GEMV
 
 where the mixer block is ``wy_lib::paged_gqa_attention_decode_block`` or
 ``wy_lib::gdn_decode_block`` (``fused_mixers=True``) or the reference's op
