@@ -175,7 +175,11 @@ def ptr(t):
 
 def stream(device: torch.device) -> int:
     """The raw handle of torch's current stream (the value of
-    ``torch.cuda.current_stream(device).cuda_stream``, without the object)."""
+    ``torch.cuda.current_stream(device).cuda_stream``, without the object).
+    Refuses a device that is no GPU, as that does: every launch passes through
+    here, and a kernel given host addresses would fault."""
+    if device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {device}")
     idx = device.index
     return torch._C._cuda_getCurrentRawStream(
         torch.cuda.current_device() if idx is None else idx)
@@ -201,8 +205,9 @@ _WORKSPACES: dict = {}
 
 def stream_workspace(device, tag: str, nbytes: int) -> torch.Tensor:
     dev = device if isinstance(device, torch.device) else torch.device(device)
+    handle = stream(dev)
     idx = dev.index if dev.index is not None else torch.cuda.current_device()
-    key = (idx, torch._C._cuda_getCurrentRawStream(idx), tag)
+    key = (idx, handle, tag)
     bufs = _WORKSPACES.get(key)
     if bufs is None:
         bufs = _WORKSPACES.setdefault(key, [])

@@ -503,3 +503,26 @@ def test_multi_instruction_asm_outputs_are_early_clobber():
             outs = re.findall(r'"(=[^"]*)"', parts[1])
             for o in outs:
                 assert o.startswith("=&"), (f.name, body[:80], o)
+
+
+def test_host_tensors_never_reach_a_launch(pkg, monkeypatch):
+    """Plain functions (no dispatcher in front) and ops given one host tensor
+    among GPU ones end at the stream lookup, which takes GPU devices only."""
+    lib = pkg._lib
+    calls = []
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda i: 7 + i)
+    monkeypatch.setattr(lib, "call", lambda name, *a: calls.append(name))
+    assert lib.stream(torch.device("cuda")) == 7 and lib.stream(torch.device("cuda:2")) == 9
+    for dev in ("cpu", "meta"):
+        with pytest.raises(ValueError, match="cuda device"):
+            lib.stream(torch.device(dev))
+        with pytest.raises(ValueError, match="cuda device"):
+            lib.stream_workspace(torch.device(dev), "host", 64)
+    q, v = torch.zeros(8, 2, 128, dtype=torch.bfloat16), torch.zeros(8, 2, 128, dtype=torch.bfloat16)
+    beta = torch.zeros(8, 2)
+    with pytest.raises(ValueError, match="cuda device"):
+        pkg.gdn_recurrent_prefill.gdn_prefill_sequential_into(
+            q, q, v, beta, beta, torch.tensor([0, 8], dtype=torch.int32),
+            torch.zeros(1, 2, 128, 128))
+    assert not calls
