@@ -434,11 +434,13 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
       if constexpr (!kState) put_row(L.Q, row, rq[i]);
     }
     if (wave == 3) {
-      // G in units of log2, summed in fp64.  A factor below 2^-149 is 0 in
-      // fp32: the clamp changes no factor and keeps differences of G finite
-      // where g = -inf (NaN passes).
+      // G in units of log2, summed in fp64.  The clamp keeps differences of G
+      // finite where g = -inf (NaN passes) and lies so low that what it clears
+      // stays cleared: later tokens' growth inside the chunk is at most 31
+      // factors below 2^128 (a larger one is infinite), and 2^(-8192 + 3968)
+      // is 0.  The fp32 pair holds 32 clamped tokens' sum to 2^-31.
       const double g2 = double(rg) * 1.4426950408889634074;
-      const double G = half_prefix(lane < nval ? (g2 < -160.0 ? -160.0 : g2) : 0.0);
+      const double G = half_prefix(lane < nval ? (g2 < -8192.0 ? -8192.0 : g2) : 0.0);
       const double G0 = lane_of(G, 31), G1 = lane_of(G, 63), Gl = lane < 32 ? G0 : G1;
       const float gh = float(G);
       L.Gh[lane] = gh;

@@ -124,6 +124,20 @@ def test_full_decay_and_growth(pkg, dev):
     assert rel(out, o64) < 2 ** -9 and rel(st, s64[0]) < 1e-6
 
 
+def test_growth_after_full_decay_brings_nothing_back(pkg, dev):
+    """What a factor exp(-400) cleared stays cleared when later tokens of the
+    same chunk grow the state by exp(80) (beta = 0 there: the state is zero)."""
+    T = 100
+    q, k, v, beta, g = inputs(T, dev, 13, 0.2)
+    g[37] = -400.0
+    beta[37:60] = 0.0
+    g[40:42] = 40.0
+    out, st = pkg.gdn_recurrent_prefill_sequential(q, k, v, beta, g)
+    o64, s64 = recurrence64(q, k, v, beta, g, [T])
+    assert (out[37:60] == 0).all()
+    assert rel(out, o64) < 2 ** -9 and rel(st, s64[0]) < 1e-6
+
+
 def test_graph_replays_and_other_stream(pkg, dev):
     lens = [SEG + 40, 77]
     args = inputs(sum(lens), dev, 5, 0.05)
