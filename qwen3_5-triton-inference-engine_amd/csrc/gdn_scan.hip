@@ -36,6 +36,13 @@
 // a sequence is cut depends on its own length alone, so a sequence gives the
 // same bits in every batch.
 //
+// Values that are not finite (infinities and NaN in the inputs, sums past
+// FLT_MAX): the products spread them further than the recurrence does, and a
+// cut infinity is NaN.  They are kept out of earlier tokens' and other
+// columns' results, and a wavefront that met one walks its columns once more
+// token by token, putting the recurrence's own value wherever its output or
+// state is not finite.
+//
 // What bounds it: a chunk is 96 MFMAs of 32 cycles and ~750 VALU operations
 // (cutting fp32 values is most of them) per wavefront, and T's chain (~4000
 // cycles per group) holds up the workgroup's four; two workgroups per CU fill
@@ -78,6 +85,7 @@ struct ScanLds {
                               // zero one
   float Gh[kG], Gl[kG], beta[kG];
   float eG[kG], E[kG], eL[4];
+  int wild;   // a value of A was not finite
 };
 static_assert(sizeof(ScanLds) <= 80 * 1024, "two workgroups per CU");
 static_assert(offsetof(ScanLds, T) % 16 == 0 && offsetof(ScanLds, A) % 16 == 0 &&
@@ -279,6 +287,154 @@ __device__ __forceinline__ u32x4_t gather8(const bf16_t *p, int64_t stride) {
   return w;
 }
 
+// ---- the recurrence token by token: lane = kg + 16 cg holds key rows 8 kg ..
+// + 7 of NC value columns, so every reduction stays inside a 16-lane DPP row.
+
+// One token's inputs as loaded (bf16 bits, fp32 g / beta): the unpack happens
+// at the step, so later tokens' loads stay in flight while a step runs.  g and
+// beta are read through VGPR addresses: vector loads complete in order, a wait
+// on a scalar load is a wait on all.
+template <int NC>
+struct TokenRaw {
+  u32x4_t k, q;
+  uint32_t v[NC / 2];
+  float g, beta;
+};
+typedef const __attribute__((address_space(1))) float gfloat_t;
+
+template <bool kContig, int NC>
+__device__ __forceinline__ void load_token_raw(const GdnArgs &a, int64_t t, int h, int kg, int col,
+                                               TokenRaw<NC> &r) {
+  const bf16_t *kp = a.k + t * a.k_t + h * a.k_h + kg * kRows * a.k_d;
+  const bf16_t *qp = a.q + t * a.q_t + h * a.q_h + kg * kRows * a.q_d;
+  const bf16_t *vp = a.v + t * a.v_t + h * a.v_h + col * a.v_d;
+  if constexpr (kContig) {
+    r.k = ld16(kp);
+    r.q = ld16(qp);
+    if constexpr (NC == 2) {
+      r.v[0] = *reinterpret_cast<const uint32_t *>(vp);
+    } else {
+#pragma unroll
+      for (int e = 0; e < NC / 4; ++e) {   // rows of v are aligned to 8 bytes
+        const u32x2_t w = *reinterpret_cast<const u32x2_t *>(vp + 4 * e);
+        r.v[2 * e] = w[0];
+        r.v[2 * e + 1] = w[1];
+      }
+    }
+  } else {
+    r.k = gather8(kp, a.k_d);
+    r.q = gather8(qp, a.q_d);
+#pragma unroll
+    for (int e = 0; e < NC / 2; ++e)
+      r.v[e] = uint32_t(vp[2 * e * a.v_d]) | (uint32_t(vp[(2 * e + 1) * a.v_d]) << 16);
+  }
+  gfloat_t *gp = (gfloat_t *)(a.g + t * a.g_t + h * a.g_h);
+  gfloat_t *bp = (gfloat_t *)(a.beta + t * a.beta_t + h * a.beta_h);
+  asm volatile("" : "+v"(gp), "+v"(bp));
+  r.g = *gp;
+  r.beta = *bp;
+}
+
+// One step on a lazily decayed state: the true state is c * s.  The decay only
+// scales c; the reductions use s and are scaled by c, the rank-1 update adds
+// k (delta / c).  When c drops below 2^-32 it is folded into s first (c = 0, a
+// full decay, clears s).
+template <int NC>
+__device__ __forceinline__ void step_scaled(float (&s)[kRows][NC], float &c, const TokenRaw<NC> &in,
+                                            float (&o)[NC]) {
+  float k[kRows], q[kRows];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    k[2 * e] = bf16_lo(in.k[e]);
+    k[2 * e + 1] = bf16_hi(in.k[e]);
+    q[2 * e] = bf16_lo(in.q[e]);
+    q[2 * e + 1] = bf16_hi(in.q[e]);
+  }
+  c *= __expf(in.g);
+  if (c < 0x1p-32f) {   // uniform: c depends on the token only
+#pragma unroll
+    for (int i = 0; i < kRows; ++i)
+#pragma unroll
+      for (int j = 0; j < NC; ++j) s[i][j] *= c;
+    c = 1.f;
+  }
+  float mem[NC], qs[NC], qk = 0.f;
+#pragma unroll
+  for (int j = 0; j < NC; ++j) mem[j] = qs[j] = 0.f;
+#pragma unroll
+  for (int i = 0; i < kRows; ++i) {
+    qk = __fmaf_rn(q[i], k[i], qk);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      mem[j] = __fmaf_rn(k[i], s[i][j], mem[j]);
+      qs[j] = __fmaf_rn(q[i], s[i][j], qs[j]);
+    }
+  }
+  qk = sum16(qk);
+  const float inv_c = __builtin_amdgcn_rcpf(c);   // 1 ulp: only scales the update
+  float dsc[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    const float vj = (j & 1) ? bf16_hi(in.v[j / 2]) : bf16_lo(in.v[j / 2]);
+    const float delta = in.beta * (vj - c * sum16(mem[j]));
+    o[j] = __fmaf_rn(qk, delta, c * sum16(qs[j]));
+    dsc[j] = delta * inv_c;
+  }
+#pragma unroll
+  for (int i = 0; i < kRows; ++i)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) s[i][j] = __fmaf_rn(k[i], dsc[j], s[i][j]);
+}
+
+// The wavefront's 4 NC columns from col0 over tokens [0, t_hi) of the sequence
+// at s0.  Where the chunks' output from token t_lo on, or the
+// state they left at sp (null: not the last segment), is not finite, the
+// walk's takes its place.
+template <bool kContig, int NC>
+__device__ __forceinline__ void walk_not_finite(const GdnArgs &a, int s0, int t_lo, int t_hi,
+                                                int h, int col0, int lane, float *sp) {
+  const int kg = lane & 15, col = col0 + NC * (lane >> 4);
+  float s[kRows][NC], c = 1.f;
+#pragma unroll
+  for (int i = 0; i < kRows; ++i)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) s[i][j] = 0.f;
+  for (int t = 0; t < t_hi; ++t) {
+    TokenRaw<NC> in;
+    load_token_raw<kContig, NC>(a, s0 + t, h, kg, col, in);
+    float o[NC];
+    step_scaled<NC>(s, c, in, o);
+    if (t < t_lo) continue;
+    bf16_t *op = a.out + int64_t(s0 + t) * a.o_t + h * a.o_h + col * a.o_d;
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+      if ((op[j * a.o_d] & 0x7f80) == 0x7f80) op[j * a.o_d] = bf16_t(f32_to_bf16_bits(o[j]));
+  }
+  if (sp == nullptr) return;
+#pragma unroll
+  for (int i = 0; i < kRows; ++i)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      float *p = sp + (kg * kRows + i) * a.s_k + col + j;
+      if (!(fabsf(*p) <= kMaxFinite)) *p = c * s[i][j];
+    }
+}
+
+// The kernel's first argument, read from the argument segment where it is used,
+// and the lane, counted there (held in registers through the chunks, they would
+// make others spill).
+__device__ __forceinline__ GdnArgs args_again() {
+  auto p = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  GdnArgs a;
+  __builtin_memcpy(&a, (const void *)p, sizeof(a));
+  return a;
+}
+__device__ __forceinline__ int lane_again() {
+  const int all = opaque(-1);
+  return __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0));
+}
+
 // kState: a non-last segment's state (and homogeneous solution) only.
 template <bool kContig, bool kState>
 __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int token_num, int batch,
@@ -316,6 +472,19 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
   const int t_lo = slots == 0 ? 0 : seg * kSeg;
   const int t_hi = slots == 0 ? len : min(len, t_lo + kSeg);
   const int col = (hom ? 0 : vb * 128) + wave * kWCols + lr;
+
+  // Where the state goes, and the distance of its rows: formed here, not by
+  // loads of the arguments in front of the stores.
+  float *dst = nullptr;
+  int64_t row = a.s_k;
+  if constexpr (kState) {
+    const Seg blk = seg_block(ws, slot0 + seg, h, a.heads, a.dv);
+    dst = hom ? blk.hom : blk.state;
+    row = hom ? kDK : a.dv;
+  } else if (seg == nseg - 1) {
+    dst = a.state + b * a.s_b + h * a.s_h;
+  }
+  asm volatile("" : "+s"(dst), "+s"(row));
 
   f32x16_t S[4];
 #pragma unroll
@@ -388,6 +557,8 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
     *reinterpret_cast<u32x2_t *>(&dst[row][kslot + 8]) = u32x2_t{x[2], x[3]};
   };
 
+  if (tid == 0) L.wild = 0;
+  bool wild = false;   // this wavefront met a value that is not finite
   // the block of T above the diagonal is zero and never written again
   for (int i = tid; i < 2 * 3 * 16 * 4; i += 256)
     *reinterpret_cast<u32x2_t *>(&L.T[i / 192][i / 64 % 3][i / 4 % 16][16 + 4 * (i % 4)]) =
@@ -446,7 +617,7 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
       L.Gh[lane] = gh;
       L.Gl[lane] = float(G - double(gh));
       // a beta that is not finite makes its row of v - k S (through eG) not
-      // finite, and so the column from this token on; T itself stays finite
+      // finite, and so the columns from this token on; T itself stays finite
       const bool fine = fabsf(rb) <= kMaxFinite;
       L.beta[lane] = lane < nval && fine ? rb : 0.f;
       L.eG[lane] = lane >= nval || fine ? __builtin_amdgcn_exp2f(gh) : __builtin_nanf("");
@@ -560,6 +731,7 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
             D = __builtin_amdgcn_mfma_f32_16x16x4f32(x11[e], P[e], D, 0, 0, 0);
           *reinterpret_cast<f32x4_t *>(&Lt[(16 + t16) * kLP + 4 * q]) = -D;
         } else {
+          float nans = 0.f;
 #pragma unroll
           for (int s = 0; s < 2; ++s) {
             float x[8];
@@ -575,10 +747,13 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
                                           acc[8 * s + 4 * q2 + e]
                                     : 0.f;
             }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) nans += x[e];
             const Pieces p = cut8(x);
 #pragma unroll
             for (int n = 0; n < 3; ++n) st16(&L.A[cc][n][lr][16 * s + 8 * hf], p.p[n]);
           }
+          if (__ballot(!(fabsf(nans) <= kMaxFinite)) != 0) L.wild = 1;
         }
       }
     }
@@ -685,12 +860,12 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
       // Row 31 of the product sees every row of R: where it is not finite, a
       // value that is not finite sits in this column of R from some token
       // t_bad on, and 0 x inf has spread it to the rows before as well.  Those
-      // are formed again without it; from t_bad on the column is NaN, as in
-      // the token-by-token recurrence.
+      // are formed again without it; from t_bad on the column is set to NaN,
+      // which the walk at the end replaces.
       int t_bad = kC;
-      const bool wild = !(fabsf(delta[15]) <= kMaxFinite) && hf == 1;
-      const bool any = __ballot(wild) != 0;
+      const bool any = __ballot(!(fabsf(delta[15]) <= kMaxFinite) && hf == 1) != 0;
       if (any) {
+        wild = true;
 #pragma unroll
         for (int r = 15; r >= 0; --r)
           if (!(fabsf(R[r]) <= kMaxFinite)) t_bad = (r & 3) + 8 * (r >> 2) + 4 * hf;
@@ -703,6 +878,8 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
       // out = exp(G) q S + A delta
       if constexpr (!kState) {
         const f32x16_t o = apply(L.A[cc], Ao, delta, lr, hf, qs);
+        // (row 31 of this product sees every row of delta)
+        wild |= __ballot(!(fabsf(o[15]) <= kMaxFinite) && hf == 1) != 0;
         bf16_t *op = a.out + tb * a.o_t + h * a.o_h;
         const int pitch = opaque(int(a.o_t) * 2);
         const auto rs = rows_rsrc(op, pitch, nv, a.dv * 2);
@@ -768,17 +945,8 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
     __syncthreads();   // the next group rewrites the LDS
   }
 
-  float *dst = nullptr;
-  int64_t row = a.s_k;
-  if constexpr (kState) {
-    const Seg blk = seg_block(ws, slot0 + seg, h, a.heads, a.dv);
-    dst = hom ? blk.hom : blk.state;
-    row = hom ? kDK : a.dv;
-  } else if (seg == nseg - 1) {
-    dst = a.state + b * a.s_b + h * a.s_h;
-  }
-  if (dst == nullptr) return;
-  if (kContig || kState) {
+  if (dst == nullptr) {
+  } else if (kContig || kState) {
     const int pitch = opaque(int(row) * 4);
     const auto rs = rows_rsrc(dst, pitch, kDK, (hom ? kDK : a.dv) * 4);
 #pragma unroll
@@ -794,6 +962,21 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
 #pragma unroll
       for (int r = 0; r < 16; ++r)
         dst[(32 * rt + (r & 3) + 8 * (r >> 2) + 4 * hf) * row + col] = S[rt][r];
+  }
+  if constexpr (!kState) {
+    // (behind the stores, which take longer)
+    float z[4] = {0.f, 0.f, 0.f, 0.f};   // NaN unless all of S is finite
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) z[rt] = __fmaf_rn(S[rt][r], 0.f, z[rt]);
+    wild |= __ballot((z[0] + z[1]) + (z[2] + z[3]) != 0.f) != 0;
+    if (t_lo < t_hi) wild |= __builtin_amdgcn_readfirstlane(L.wild) != 0;
+    if (wild) {
+      __threadfence_block();   // other lanes' results are read back
+      walk_not_finite<kContig, 8>(args_again(), s0, t_lo, t_hi, h, vb * 128 + wave * kWCols,
+                                  lane_again(), dst);
+    }
   }
 }
 

@@ -112,6 +112,73 @@ def test_nan_stays_behind_its_token(pkg, dev, what, t):
         assert bad[t:].all() and torch.isnan(st[0, 0]).all()
 
 
+def step_recurrence64(q, k, v, beta, g):
+    """One sequence with out = q S_decayed + (q k) delta, the kernels' form (at
+    an infinite delta it keeps a sign that q S_new, a sum over key rows of both
+    signs, has not)."""
+    outs = []
+    q, k, v, beta, g = (x.double().cpu() for x in (q, k, v, beta, g))
+    s = torch.zeros(H, D, D, dtype=torch.float64)
+    for t in range(q.shape[0]):
+        s = s * torch.exp(g[t])[:, None, None]
+        d = beta[t][:, None] * (v[t] - (k[t][:, :, None] * s).sum(1))
+        outs.append((q[t][:, :, None] * s).sum(1) + (q[t] * k[t]).sum(1)[:, None] * d)
+        s = s + k[t][:, :, None] * d[:, None, :]
+    return torch.stack(outs), s
+
+
+def same_class(x, y):
+    x, y = x.double().cpu(), y.double().cpu()
+    assert torch.equal(torch.isnan(x), torch.isnan(y))
+    inf = torch.isinf(y)
+    assert torch.equal(torch.isinf(x), inf) and torch.equal(x[inf], y[inf])
+    fine = torch.isfinite(y)
+    torch.testing.assert_close(x[fine], y[fine], atol=2e-2, rtol=2e-2)   # (two bf16 roundings)
+
+
+@pytest.mark.parametrize("what", ["v", "k", "q", "beta"])
+@pytest.mark.parametrize("t", [0, 20, 40, SEG + 3, SEG + 63])
+def test_infinity_as_in_the_recurrence(pkg, dev, what, t):
+    """An infinite input gives the recurrence's infinities, signs included, at
+    its own token and in the state, and changes nothing else."""
+    T = SEG + 64
+    args = dict(zip(("q", "k", "v", "beta", "g"), inputs(2 * T, dev, 5, 0.1)))
+    cu = cu_of([T, T], dev)
+    want, want_st = pkg.gdn_recurrent_prefill_sequential(*args.values(), cu)
+    x = args[what].clone()
+    if x.ndim == 3:
+        x[t, 0, 5] = float("inf") if t % 2 else -float("inf")
+    else:
+        x[t, 0] = float("inf")
+    args[what] = x
+    out, st = pkg.gdn_recurrent_prefill_sequential(*args.values(), cu)
+    o64, s64 = step_recurrence64(*(y[:T] for y in args.values()))
+    same_class(out[:T], o64)
+    same_class(st[0], s64)
+    assert torch.equal(out[:t], want[:t]) and torch.equal(out[T:], want[T:])
+    assert torch.equal(out[:, 1], want[:, 1]) and torch.equal(st[1], want_st[1])
+    if what == "v":
+        assert torch.isinf(out[t, 0, 5])
+        keep = torch.arange(D, device=dev) != 5
+        assert torch.equal(out[:, 0, keep], want[:, 0, keep])
+
+
+def test_overflow_reaches_no_earlier_token(pkg, dev):
+    """beta v past FLT_MAX at token 40 from finite inputs: its column alone,
+    from its own token on."""
+    T = 60
+    q, k, v, beta, g = inputs(T, dev, 15, 0.1)
+    v[40, 0, 5] = 3e38
+    beta[40, 0] = 4.0
+    out, st = pkg.gdn_recurrent_prefill_sequential(q, k, v, beta, g)
+    o64, s64 = step_recurrence64(q, k, v, beta, g)
+    fine = torch.ones(T, H, D, dtype=torch.bool)
+    fine[40:, 0, 5] = False
+    assert torch.equal(torch.isfinite(out).cpu(), fine)
+    same_class(out.cpu()[fine], o64[fine])
+    assert torch.isfinite(st[0, :, :5]).all() and torch.isfinite(st[1]).all()
+
+
 def test_full_decay_and_growth(pkg, dev):
     """g = -inf clears the state; g > 0 grows it."""
     T = 100
