@@ -494,6 +494,21 @@ int wy_gdn_prefill_varlen(const void *q, const int64_t *q_strides, const void *k
                           int token_num, int batch, int num_heads, int key_dim, int value_dim,
                           float *workspace, int64_t workspace_bytes, void *stream);
 
+/*
+ * wy_gdn_prefill_varlen for a caller that knows the longest sequence's length:
+ * max_seqlen tokens at least (0: unknown).  Where it is at most 8 the whole
+ * batch is walked token by token in one light launch; where the workspace size
+ * for max_seqlen tokens is 0, none is needed.  Same results either way.
+ */
+int wy_gdn_prefill_varlen_max(const void *q, const int64_t *q_strides, const void *k,
+                              const int64_t *k_strides, const void *v, const int64_t *v_strides,
+                              const float *beta, const int64_t *beta_strides, const float *g,
+                              const int64_t *g_strides, void *out, const int64_t *out_strides,
+                              float *state, const int64_t *state_strides,
+                              const int32_t *cu_seqlens, int token_num, int max_seqlen, int batch,
+                              int num_heads, int key_dim, int value_dim, float *workspace,
+                              int64_t workspace_bytes, void *stream);
+
 /* Workspace size of wy_gdn_prefill_varlen (0: none needed). */
 int64_t wy_gdn_prefill_varlen_workspace_bytes(int token_num, int num_heads, int value_dim);
 

@@ -70,6 +70,9 @@ _SIGNATURES = {
     "wy_gdn_prefill_varlen": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp,
                               _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _i, _i, _i, _i, _i, _vp,
                               _i64, _vp],
+    "wy_gdn_prefill_varlen_max": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp,
+                              _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _i, _i, _i, _i, _i, _i, _vp,
+                              _i64, _vp],
     "wy_depthwise_causal_conv4_decode": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp,
                                          _c_i64p, _i, _i, _vp],
     "wy_gdn_qk_norm_gates": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _vp,

@@ -50,8 +50,8 @@
 // recurrence alone, against one wavefront per 16 columns walking token by
 // token): 32 x 128 tokens 200 -> 43 us, 24 prompts of 22..4096 tokens (23.8k)
 // 3.10 ms -> 0.47 ms, one prompt of 1000 tokens 304 -> 142 us, one of 5003
-// 287 (chunk ops of csrc/gdn_chunk.hip) -> 189 us; one of 16 tokens 7.8 -> 9.0
-// us, the chunk's fixed cost.  Segment length (same cases, us; 128 / 256 / 512
+// 287 (chunk ops of csrc/gdn_chunk.hip) -> 189 us; one of 9 to 16 tokens 6.4 to
+// 8.6 -> 9.5 us, the chunk's fixed cost.  Segment length (same cases, us; 128 / 256 / 512
 // / 1024 tokens): 23.8k mixed 710 / 557 / 470 / 402, 5003 250 / 194 / 189 /
 // 288, 1000 68 / 85 / 142 / 153.
 #include "gdn_common.h"
@@ -68,6 +68,24 @@ constexpr int kG = 64;        // tokens staged together (two chunks)
 #endif
 constexpr int kSeg = WY_GDN_SEG;   // tokens per segment
 static_assert(kSeg % kG == 0, "segments hold whole groups");
+// Sequences of at most kWalk tokens are walked token by token: a chunk costs
+// the same whatever it holds.  One prompt, us a launch, walked by
+// gdn_walk_kernel / as a chunk: 1 token 3.6 / 9.5, 8 tokens 6.3 / 9.5, 16
+// tokens 8.6 / 9.5.  In batches the chunk wins earlier: 16 sequences of 8
+// tokens 13.4 / 12.3, of 16 tokens 19.6 / 12.6, 64 of 8 32 / 29, of 16 55 / 37;
+// the line is one for all, so that a sequence gives the same bits in every
+// batch.
+#ifndef WY_GDN_WALK
+#define WY_GDN_WALK 8
+#endif
+constexpr int kWalk = WY_GDN_WALK;
+// A batch of such sequences alone (known from the longest one's length, or from
+// the token total) is gdn_walk_kernel's up to kWalkBatch sequences.  Inside
+// the scan kernel, 8 columns a lane, a short sequence waits on its chains where
+// the chip is not full, and saves the re-read q and k where it is: 64 sequences
+// of 4 tokens 22 us / 28 inside, 256 of 4 80 / 105, 1024 of 4 490 / 404, 4096
+// of one 1.9 ms / 1.2.
+constexpr int kWalkBatch = 512;
 constexpr int kKP = kDK + 8;  // LDS row pitch of k and q (bf16): 16-byte reads of 16 rows fill all banks
 constexpr int kTP = kC + 8;   // of T and A
 constexpr int kLP = kC + 4;   // of L (fp32)
@@ -254,6 +272,19 @@ __device__ __forceinline__ bool find_segment(const int32_t *cu, int token_num, i
   return false;
 }
 
+// Non-last segments in the sequences before b (of a batch with cu_seqlens).
+__device__ __forceinline__ int slots_before(const int32_t *cu, int b, int lane) {
+  int n = 0;
+  for (int b0 = 0; b0 < b; b0 += 64) {
+    const int i = b0 + lane;
+    int x = i < b ? seg_count(cu[i + 1] - cu[i]) - 1 : 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+    n += x;
+  }
+  return n;
+}
+
 // Two workspace blocks per (slot, head): the state after the segment (value
 // columns: dv of them) and its homogeneous solution P [128][128].
 struct Seg {
@@ -287,6 +318,21 @@ __device__ __forceinline__ u32x4_t gather8(const bf16_t *p, int64_t stride) {
   return w;
 }
 
+// The kernel's first argument, read from the argument segment where it is used,
+// and the lane, counted there (held in registers through the chunks, they would
+// make others spill).
+__device__ __forceinline__ GdnArgs args_again() {
+  auto p = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  GdnArgs a;
+  __builtin_memcpy(&a, (const void *)p, sizeof(a));
+  return a;
+}
+__device__ __forceinline__ int lane_again() {
+  const int all = opaque(-1);
+  return __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0));
+}
+
 // ---- the recurrence token by token: lane = kg + 16 cg holds key rows 8 kg ..
 // + 7 of NC value columns, so every reduction stays inside a 16-lane DPP row.
 
@@ -297,7 +343,7 @@ __device__ __forceinline__ u32x4_t gather8(const bf16_t *p, int64_t stride) {
 template <int NC>
 struct TokenRaw {
   u32x4_t k, q;
-  uint32_t v[NC / 2];
+  uint32_t v[(NC + 1) / 2];
   float g, beta;
 };
 typedef const __attribute__((address_space(1))) float gfloat_t;
@@ -311,8 +357,8 @@ __device__ __forceinline__ void load_token_raw(const GdnArgs &a, int64_t t, int 
   if constexpr (kContig) {
     r.k = ld16(kp);
     r.q = ld16(qp);
-    if constexpr (NC == 2) {
-      r.v[0] = *reinterpret_cast<const uint32_t *>(vp);
+    if constexpr (NC == 1) {
+      r.v[0] = vp[0];
     } else {
 #pragma unroll
       for (int e = 0; e < NC / 4; ++e) {   // rows of v are aligned to 8 bytes
@@ -324,6 +370,7 @@ __device__ __forceinline__ void load_token_raw(const GdnArgs &a, int64_t t, int 
   } else {
     r.k = gather8(kp, a.k_d);
     r.q = gather8(qp, a.q_d);
+    r.v[0] = vp[0];
 #pragma unroll
     for (int e = 0; e < NC / 2; ++e)
       r.v[e] = uint32_t(vp[2 * e * a.v_d]) | (uint32_t(vp[(2 * e + 1) * a.v_d]) << 16);
@@ -386,6 +433,74 @@ __device__ __forceinline__ void step_scaled(float (&s)[kRows][NC], float &c, con
     for (int j = 0; j < NC; ++j) s[i][j] = __fmaf_rn(k[i], dsc[j], s[i][j]);
 }
 
+// A whole sequence from a zero state, the wavefront's 4 NC columns from col0.
+// The sums keep one order whatever NC is: the same bits.  kAhead tokens are in flight: every load and store is
+// unconditional (a request past the end re-reads the last token, the 16 lanes of
+// a row store the same output), so a wait names exactly the token a step needs.
+template <bool kContig, int NC>
+__device__ __forceinline__ void walk(const GdnArgs &a, int s0, int len, int b, int h, int col0,
+                                     int lane) {
+  constexpr int kAhead = NC == 1 ? 4 : 2;
+  const int kg = lane & 15, col = col0 + NC * (lane >> 4);
+  float s[kRows][NC], c = 1.f;
+#pragma unroll
+  for (int i = 0; i < kRows; ++i)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) s[i][j] = 0.f;
+  if (len > 0) {
+    auto put = [&](int t, const float (&o)[NC]) {
+      bf16_t *op = a.out + int64_t(s0 + t) * a.o_t + h * a.o_h + col * a.o_d;
+      if constexpr (!kContig || NC == 1) {
+#pragma unroll
+        for (int j = 0; j < NC; ++j) op[j * a.o_d] = bf16_t(f32_to_bf16_bits(o[j]));
+      } else {
+#pragma unroll
+        for (int j = 0; j < NC; j += 4)   // rows of out are aligned to 8 bytes
+          *reinterpret_cast<u32x2_t *>(op + j) =
+              u32x2_t{pack_bf16x2(o[j], o[j + 1]), pack_bf16x2(o[j + 2], o[j + 3])};
+      }
+    };
+    TokenRaw<NC> in[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      load_token_raw<kContig, NC>(a, s0 + min(u, len - 1), h, kg, col, in[u]);
+    const int whole = len - len % kAhead;
+    for (int t = 0; t < whole; t += kAhead) {
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        float o[NC];
+        step_scaled<NC>(s, c, in[u], o);
+        put(t + u, o);
+        load_token_raw<kContig, NC>(a, s0 + min(t + u + kAhead, len - 1), h, kg, col, in[u]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead - 1; ++u)
+      if (whole + u < len) {
+        float o[NC];
+        step_scaled<NC>(s, c, in[u], o);
+        put(whole + u, o);
+      }
+  }
+  float *sp = a.state + b * a.s_b + h * a.s_h + int64_t(kg * kRows) * a.s_k + col;
+#pragma unroll
+  for (int i = 0; i < kRows; ++i)
+#pragma unroll
+    for (int j = 0; j < NC; ++j) sp[i * a.s_k + j] = c * s[i][j];
+}
+
+// A batch of sequences of at most kWalk tokens each: one wavefront to 4 NC
+// columns of a (sequence, head), sequence fastest.
+template <bool kContig, int NC>
+__global__ __launch_bounds__(64) void gdn_walk_kernel(const GdnArgs a, int token_num, int batch) {
+  const int b = blockIdx.x % batch;
+  const int h = (blockIdx.x / batch) % a.heads;
+  const int col0 = blockIdx.x / (batch * a.heads) * 4 * NC;
+  const int s0 = seq_start(a.cu_seqlens, token_num, b);
+  walk<kContig, NC>(a, s0, seq_start(a.cu_seqlens, token_num, b + 1) - s0, b, h, col0,
+                    threadIdx.x);
+}
+
 // The wavefront's 4 NC columns from col0 over tokens [0, t_hi) of the sequence
 // at s0.  Where the chunks' output from token t_lo on, or the
 // state they left at sp (null: not the last segment), is not finite, the
@@ -420,21 +535,6 @@ __device__ __forceinline__ void walk_not_finite(const GdnArgs &a, int s0, int t_
     }
 }
 
-// The kernel's first argument, read from the argument segment where it is used,
-// and the lane, counted there (held in registers through the chunks, they would
-// make others spill).
-__device__ __forceinline__ GdnArgs args_again() {
-  auto p = __builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(p));
-  GdnArgs a;
-  __builtin_memcpy(&a, (const void *)p, sizeof(a));
-  return a;
-}
-__device__ __forceinline__ int lane_again() {
-  const int all = opaque(-1);
-  return __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0));
-}
-
 // kState: a non-last segment's state (and homogeneous solution) only.
 template <bool kContig, bool kState>
 __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int token_num, int batch,
@@ -453,10 +553,18 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
   const int item = blockIdx.x / (a.heads * cols);
   const bool hom = kState && vb == vblocks;
   int b, seg = 0, slot0 = 0;
+  // A search costs a memory round trip for every 64 sequences.  Larger batches
+  // list the non-last segments (few, and the longest walks) first and then every
+  // sequence's last one, whose sequence is the item's number: 4096 sequences of
+  // 8 tokens searched for took 4.0 ms, listed 2.2.
+  const bool listed = !kState && batch > 64 && item >= slots;
   if (slots == 0) {
     b = item;   // no segments: one item per sequence
     if (b >= batch) return;
-  } else if (!find_segment(a.cu_seqlens, token_num, batch, item, kState, b, seg, slot0)) {
+  } else if (listed) {
+    b = item - slots;
+  } else if (!find_segment(a.cu_seqlens, token_num, batch, item, kState || batch > 64, b, seg,
+                           slot0)) {
     return;
   }
   // the same in every lane: pointers and buffer resources built from them
@@ -466,7 +574,17 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
   slot0 = __builtin_amdgcn_readfirstlane(slot0);
   const int s0 = seq_start(a.cu_seqlens, token_num, b);
   const int len = seq_start(a.cu_seqlens, token_num, b + 1) - s0;
+  if constexpr (!kState) {
+    if (len <= kWalk) {
+      walk<kContig, 8>(args_again(), s0, len, b, h, vb * 128 + wave * kWCols, lane_again());
+      return;
+    }
+  }
   const int nseg = slots == 0 ? 1 : seg_count(len);
+  if (listed && nseg > 1) {
+    seg = nseg - 1;
+    slot0 = slots_before(a.cu_seqlens, b, lane);
+  }
   if (slot0 + nseg - 1 > slots) return;   // more tokens than the workspace was sized for
   if (hom && seg == 0) return;            // the first segment starts from a known (zero) state
   const int t_lo = slots == 0 ? 0 : seg * kSeg;
@@ -993,14 +1111,7 @@ __global__ __launch_bounds__(256) void gdn_fold_kernel(const int32_t *cu, int to
   const int lr = lane & 31, hf = lane >> 5;
   const int nseg = seg_count(seq_start(cu, token_num, b + 1) - seq_start(cu, token_num, b));
   if (nseg < 3) return;   // S_1 = U_0 needs no fold
-  int slot0 = 0;
-  for (int b0 = 0; b0 < b; b0 += 64) {
-    const int i = b0 + lane;
-    int x = i < b ? seg_count(cu[i + 1] - cu[i]) - 1 : 0;   // b > 0: there is a cu
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-    slot0 += x;
-  }
+  const int slot0 = slots_before(cu, b, lane);   // (b > 0: there is a cu)
   if (slot0 + nseg - 1 > slots) return;
   const int col = cb * kWCols + lr;
   const int row0 = 32 * wave + 4 * hf;
@@ -1065,6 +1176,21 @@ __global__ __launch_bounds__(256) void gdn_fold_kernel(const int32_t *cu, int to
 }
 
 template <bool kContig>
+int launch_walk(const GdnArgs &a, int token_num, int batch, hipStream_t st) {
+  // Four columns a lane fill the chip from 2048 wavefronts on; below that one
+  // a lane, whose steps are shorter chains.
+  const int64_t wide = int64_t(batch) * a.heads * (a.dv / 16);
+  const bool narrow = wide < 2048;
+  const int64_t groups = narrow ? wide * 4 : wide;
+  if (groups > 0x7fffffff) return WY_E_SHAPE;
+  if (narrow)
+    gdn_walk_kernel<kContig, 1><<<unsigned(groups), 64, 0, st>>>(a, token_num, batch);
+  else
+    gdn_walk_kernel<kContig, 4><<<unsigned(groups), 64, 0, st>>>(a, token_num, batch);
+  return wyh::launch_status();
+}
+
+template <bool kContig>
 int launch_scan(const GdnArgs &a, int token_num, int batch, float *ws, int slots, hipStream_t st) {
   const int vblocks = a.dv / 128;
   const int64_t main = int64_t(batch + slots) * a.heads * vblocks;
@@ -1103,16 +1229,13 @@ extern "C" int64_t wy_gdn_prefill_varlen_workspace_bytes(int token_num, int num_
   return slot_bound(token_num) * num_heads * kDK * (int64_t(value_dim) + kDK) * 4;
 }
 
-extern "C" int wy_gdn_prefill_varlen(const void *q, const int64_t *q_strides, const void *k,
-                                     const int64_t *k_strides, const void *v,
-                                     const int64_t *v_strides, const float *beta,
-                                     const int64_t *beta_strides, const float *g,
-                                     const int64_t *g_strides, void *out,
-                                     const int64_t *out_strides, float *state,
-                                     const int64_t *state_strides, const int32_t *cu_seqlens,
-                                     int token_num, int batch, int num_heads, int key_dim,
-                                     int value_dim, float *workspace, int64_t workspace_bytes,
-                                     void *stream) {
+extern "C" int wy_gdn_prefill_varlen_max(
+    const void *q, const int64_t *q_strides, const void *k, const int64_t *k_strides,
+    const void *v, const int64_t *v_strides, const float *beta, const int64_t *beta_strides,
+    const float *g, const int64_t *g_strides, void *out, const int64_t *out_strides,
+    float *state, const int64_t *state_strides, const int32_t *cu_seqlens, int token_num,
+    int max_seqlen, int batch, int num_heads, int key_dim, int value_dim, float *workspace,
+    int64_t workspace_bytes, void *stream) {
   GdnArgs a;
   bool contig = false;
   const int rc = gdn_setup(a, contig, q, q_strides, k, k_strides, v, v_strides, beta,
@@ -1120,9 +1243,14 @@ extern "C" int wy_gdn_prefill_varlen(const void *q, const int64_t *q_strides, co
                            num_heads, key_dim, value_dim);
   if (rc != WY_OK) return rc;
   if (!cu_seqlens && batch != 1) return WY_E_NULL;
-  if (batch < 0 || token_num < 0) return WY_E_SHAPE;
+  if (batch < 0 || token_num < 0 || max_seqlen < 0) return WY_E_SHAPE;
   if (batch == 0) return WY_OK;
   a.cu_seqlens = cu_seqlens;
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  const int bound = max_seqlen > 0 ? max_seqlen : token_num;   // 0: unknown
+  if (bound > 0 && bound <= kWalk && batch <= kWalkBatch)
+    return contig ? launch_walk<true>(a, token_num, batch, st)
+                  : launch_walk<false>(a, token_num, batch, st);
   const int64_t slots = workspace ? slot_bound(token_num) : 0;
   if (slots > 0x7fffffff / 2) return WY_E_SHAPE;
   if (slots > 0 && workspace_bytes <
@@ -1134,9 +1262,24 @@ extern "C" int wy_gdn_prefill_varlen(const void *q, const int64_t *q_strides, co
   const auto row_ok = [](int64_t t, int64_t width) { return t >= width && t < (1 << 22); };
   contig = contig && row_ok(a.q_t, kDK) && row_ok(a.k_t, kDK) && row_ok(a.v_t, a.dv) &&
            row_ok(a.o_t, a.dv) && row_ok(a.s_k, a.dv) && row_ok(a.g_t, 1) && row_ok(a.beta_t, 1);
-  const hipStream_t st = static_cast<hipStream_t>(stream);
   return contig ? launch_scan<true>(a, token_num, batch, workspace, int(slots), st)
                 : launch_scan<false>(a, token_num, batch, workspace, int(slots), st);
+}
+
+extern "C" int wy_gdn_prefill_varlen(const void *q, const int64_t *q_strides, const void *k,
+                                     const int64_t *k_strides, const void *v,
+                                     const int64_t *v_strides, const float *beta,
+                                     const int64_t *beta_strides, const float *g,
+                                     const int64_t *g_strides, void *out,
+                                     const int64_t *out_strides, float *state,
+                                     const int64_t *state_strides, const int32_t *cu_seqlens,
+                                     int token_num, int batch, int num_heads, int key_dim,
+                                     int value_dim, float *workspace, int64_t workspace_bytes,
+                                     void *stream) {
+  return wy_gdn_prefill_varlen_max(q, q_strides, k, k_strides, v, v_strides, beta, beta_strides,
+                                   g, g_strides, out, out_strides, state, state_strides,
+                                   cu_seqlens, token_num, 0, batch, num_heads, key_dim, value_dim,
+                                   workspace, workspace_bytes, stream);
 }
 
 extern "C" int wy_gdn_recurrent_prefill_sequential(

@@ -325,7 +325,7 @@ class DecodeModel:
             self.rec_states[i].copy_(state)
         else:
             core = gdn_prefill_sequential_into(qn, kn, v, beta, g, packed.cu_seqlens,
-                                               self.rec_states[i])
+                                               self.rec_states[i], packed.max_seqlen)
         conv_state_from_packed_prefill(self.conv_states[i], qkv, packed.cu_seqlens)
         normed = gdn_gated_rmsnorm(core, fused[:, 3 * HD:4 * HD].view(T, H, D), w.extra["norm"])
         return gemm_2d(normed.view(T, HD), w.out_proj)

@@ -11,6 +11,8 @@ CPU path.
 
 from __future__ import annotations
 
+from operator import sub
+
 import torch
 
 from . import _lib
@@ -41,17 +43,22 @@ def _tensor_args(q, k, v, beta, g, out, state):
     )
 
 
-def _prefill(q, k, v, beta, g, out, state, cu_seqlens):
-    """The packed prefill into ``out`` and ``state``.  The workspace (segment
-    states of sequences over 512 tokens) lives for this call."""
+def _prefill(q, k, v, beta, g, out, state, cu_seqlens, max_seqlen):
+    """The packed prefill into ``out`` and ``state``; ``max_seqlen``: the
+    longest sequence, 0 if the host does not know it.  The workspace (segment
+    states of sequences over 512 tokens, where there may be one) lives for this
+    call."""
     token_num, num_heads, key_dim = q.shape
     value_dim = v.shape[-1]
-    nbytes = _lib.load().wy_gdn_prefill_varlen_workspace_bytes(token_num, num_heads, value_dim)
+    size = _lib.load().wy_gdn_prefill_varlen_workspace_bytes
+    nbytes = size(token_num, num_heads, value_dim)
+    if nbytes and max_seqlen and not size(max_seqlen, num_heads, value_dim):
+        nbytes = 0
     ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
     _lib.call(
-        "wy_gdn_prefill_varlen", *_tensor_args(q, k, v, beta, g, out, state),
-        _lib.ptr(cu_seqlens), token_num, state.shape[0], num_heads, key_dim, value_dim,
-        _lib.ptr(ws), nbytes, _lib.stream(q.device),
+        "wy_gdn_prefill_varlen_max", *_tensor_args(q, k, v, beta, g, out, state),
+        _lib.ptr(cu_seqlens), token_num, max_seqlen, state.shape[0], num_heads, key_dim,
+        value_dim, _lib.ptr(ws), nbytes, _lib.stream(q.device),
     )
 
 
@@ -77,16 +84,20 @@ def gdn_recurrent_prefill_sequential(
     assert token_num > 0 and num_heads > 0
     if cu_seqlens is not None:
         assert cu_seqlens.dtype == torch.int32 and cu_seqlens.ndim == 1
-        assert int(cu_seqlens[-1]) == token_num, (
-            f"cu_seqlens[-1]={int(cu_seqlens[-1])} does not match the packed token count "
-            f"{token_num}"
+        ends = cu_seqlens.tolist()
+        assert ends[-1] == token_num, (
+            f"cu_seqlens[-1]={ends[-1]} does not match the packed token count {token_num}"
         )
+        # (the longest of many is not worth its host time)
+        max_seqlen = max(map(sub, ends[1:], ends), default=0) if len(ends) <= 257 else 0
         cu_seqlens = cu_seqlens.contiguous()
+    else:
+        max_seqlen = token_num
     batch = 1 if cu_seqlens is None else cu_seqlens.numel() - 1
     out = torch.empty_like(v)
     state = torch.empty((batch, num_heads, key_dim, value_dim), dtype=torch.float32,
                         device=q.device)
-    _prefill(q, k, v, beta, g, out, state, cu_seqlens)
+    _prefill(q, k, v, beta, g, out, state, cu_seqlens, max_seqlen)
     return out, (state[0] if cu_seqlens is None else state)
 
 
@@ -98,12 +109,14 @@ def _gdn_recurrent_prefill_sequential_fake(q, k, v, beta, g, cu_seqlens=None):
     return torch.empty_like(v), torch.empty(shape, dtype=torch.float32, device=q.device)
 
 
-def gdn_prefill_sequential_into(q, k, v, beta, g, cu_seqlens, state):
+def gdn_prefill_sequential_into(q, k, v, beta, g, cu_seqlens, state, max_seqlen=None):
     """The packed sequential prefill writing its final states into ``state``
     (``[B, H, DK, DV]`` fp32, e.g. a decoder's recurrent-state cache) instead
     of a new tensor, for callers that validated ``cu_seqlens`` on the host
     (``PackedBatch``): no device-to-host read of ``cu_seqlens[-1]`` and no
-    state copy.  Returns ``out [T, H, DV]`` bf16."""
+    state copy.  ``max_seqlen``, where the caller knows the longest sequence's
+    length, saves launches that a batch of short ones has no use for.  Returns
+    ``out [T, H, DV]`` bf16."""
     _check_common(q, k, v, beta, g)
     token_num, num_heads, key_dim = q.shape
     value_dim = v.shape[-1]
@@ -112,7 +125,7 @@ def gdn_prefill_sequential_into(q, k, v, beta, g, cu_seqlens, state):
     assert state.dtype == torch.float32
     assert state.shape == (batch, num_heads, key_dim, value_dim)
     out = torch.empty_like(v)
-    _prefill(q, k, v, beta, g, out, state, cu_seqlens)
+    _prefill(q, k, v, beta, g, out, state, cu_seqlens, max_seqlen or 0)
     return out
 
 

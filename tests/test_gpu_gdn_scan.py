@@ -67,7 +67,41 @@ def test_lengths_vs_recurrence(pkg, dev, lens, decay):
         o += n
 
 
-@pytest.mark.parametrize("T", [33, SEG + 70])
+# walked alone (8 tokens at most), in chunks, in segments; by the token walk's own
+# kernel (one and four columns a lane: from 128 sequences of two heads) and
+# inside the scan kernel; more than 64 sequences: listed segments; more than 512
+@pytest.mark.parametrize("lens", [
+    [1, 8, 0, 3], [8] * 40, [1, 2, 7, 8] * 33, [8, 9, 1, 40], [5] * 63 + [SEG + 1],
+    [3, 9] * 34 + [2 * SEG + 5, 0, SEG + 1, 8, 2 * SEG], [4] * 520, [4] * 130 + [600]])
+def test_short_sequences_same_bits_by_every_route(pkg, dev, lens):
+    T = sum(lens)
+    args = inputs(T, dev, 17 + T, 0.2)
+    cu = cu_of(lens, dev)
+    into = pkg.gdn_recurrent_prefill.gdn_prefill_sequential_into
+    got = []
+    for hint in (None, max(lens)):
+        st = torch.full((len(lens), H, D, D), float("nan"), device=dev)
+        got.append((into(*args, cu, st, hint), st))
+    got.append(pkg.gdn_recurrent_prefill_sequential(*args, cu))
+    for out, st in got[1:]:
+        assert torch.equal(out, got[0][0]) and torch.equal(st, got[0][1])
+    out, st = got[0]
+    o = 0
+    for b, n in enumerate(lens):
+        if n and (b < 8 or b > len(lens) - 8):
+            o1, s1 = pkg.gdn_recurrent_prefill_sequential(*(x[o:o + n] for x in args))
+            assert torch.equal(s1, st[b]) and torch.equal(o1, out[o:o + n])
+        elif n == 0:
+            assert not st[b].any()
+        o += n
+    some = [b for b, n in enumerate(lens) if 0 < n <= 9][:6]
+    starts = [sum(lens[:b]) for b in some]
+    rows = torch.cat([torch.arange(o, o + lens[b]) for b, o in zip(some, starts)]).to(dev)
+    o64, s64 = recurrence64(*(x[rows] for x in args), [lens[b] for b in some])
+    assert rel(out[rows], o64) < 2 ** -9 and rel(st[some], s64) < 1e-6
+
+
+@pytest.mark.parametrize("T", [7, 33, SEG + 70])
 def test_other_strides_same_bits(pkg, dev, T):
     q, k, v, beta, g = inputs(T, dev, T)
 
