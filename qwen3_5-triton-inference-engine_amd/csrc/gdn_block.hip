@@ -314,7 +314,14 @@ __global__ __launch_bounds__(256) void gdn_gated_rmsnorm_vec_kernel(
 // that mapping: 4096 tokens 4: 26.5 / 21.1, 8: 24.6 / 22.1, 16: 25.4 / 24.8;
 // 23772 tokens 130 / 120, 140 / 120, 136 / 126.  With 2-byte weight loads, the
 // library division and runs of 16 it took 29.3 and 137; a copy takes 15 and 108.
-template <int kRun, bool kRowsW, bool kSeq>
+//
+// Weights: rows of channels (the decode weight's transpose), 4 taps side by
+// side ([C, 4] contiguous, 64 bytes a thread), or any strides: 32 loads of 2
+// bytes, which runs of 16 tokens share where there are enough workgroups (6144
+// channels, us, runs of 4 / 16: 512 tokens 11.6 / 12.9, 1000 16.2 / 14.5, 4096
+// 51.9 / 31.9; [C, 4] contiguous 22).
+enum ConvWeights { kTapRows, kTapQuads, kTapAny };
+template <int kRun, ConvWeights kW, bool kSeq>
 __global__ __launch_bounds__(256) void conv4_prefill_vec_kernel(
     const bf16_t *__restrict__ x, int64_t x_t, const bf16_t *__restrict__ w, int64_t w_c,
     int64_t w_k, bf16_t *__restrict__ out, int64_t o_t, const int32_t *__restrict__ seq_start,
@@ -325,9 +332,12 @@ __global__ __launch_bounds__(256) void conv4_prefill_vec_kernel(
   const int t0 = run * kRun;
   if (c0 >= C || t0 >= T) return;
   u32x4_t wr[4];
-  if constexpr (kRowsW) {
+  if constexpr (kW == kTapRows) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) wr[k] = ld16(w + k * w_k + c0);
+  } else if constexpr (kW == kTapQuads) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) wr[k] = ld16(w + 4 * c0 + 8 * k);   // channels 2k, 2k + 1
   } else {
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -351,8 +361,19 @@ __global__ __launch_bounds__(256) void conv4_prefill_vec_kernel(
     win[j] = ld16(x + int64_t(t) * x_t + c0);
   }
   float wt[4][8];
+  if constexpr (kW == kTapQuads) {
 #pragma unroll
-  for (int k = 0; k < 4; ++k) unpack8(wr[k], wt[k]);
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int k = 0; k < 4; k += 2) {
+        const uint32_t two = wr[j / 2][2 * (j & 1) + k / 2];
+        wt[k][j] = bf16_lo(two);
+        wt[k + 1][j] = bf16_hi(two);
+      }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) unpack8(wr[k], wt[k]);
+  }
   // each window row is unpacked once into a rolling 4-row float window; the
   // per-row masks for rows before the sequence's start are only evaluated for
   // a token whose window reaches past it (a block-uniform branch); the pair
@@ -682,19 +703,27 @@ extern "C" int wy_depthwise_causal_conv4_prefill(const void *x, const int64_t *x
   const unsigned runs = unsigned((tokens + kConvRun - 1) / kConvRun);
   if (x_strides[1] == 1 && out_strides[1] == 1 && channels % 8 == 0 &&
       ((x_strides[0] | out_strides[0]) & 7) == 0 && wyh::aligned16(x) && wyh::aligned16(out)) {
-    const bool w_rows = w_stride_c == 1 && w_stride_k % 8 == 0 && wyh::aligned16(weight);
-    const unsigned vruns = unsigned((tokens + kConvVecRun - 1) / kConvVecRun);
     const int xb = (channels / 8 + 255) / 256;
-    auto *kernel =
-        w_rows ? (seq_start ? conv4_prefill_vec_kernel<kConvVecRun, true, true>
-                            : conv4_prefill_vec_kernel<kConvVecRun, true, false>)
-               : (seq_start ? conv4_prefill_vec_kernel<kConvVecRun, false, true>
-                            : conv4_prefill_vec_kernel<kConvVecRun, false, false>);
-    const unsigned tiles = unsigned(xb) * vruns;
-    kernel<<<(tiles + 7) / 8 * 8, 256, 0, static_cast<hipStream_t>(stream)>>>(
-        static_cast<const bf16_t *>(x), x_strides[0], static_cast<const bf16_t *>(weight),
-        w_stride_c, w_stride_k, static_cast<bf16_t *>(out), out_strides[0], seq_start, tokens,
-        channels, xb);
+    const auto launch = [&](auto kernel, int run) {
+      const unsigned tiles = unsigned(xb) * unsigned((tokens + run - 1) / run);
+      kernel<<<(tiles + 7) / 8 * 8, 256, 0, static_cast<hipStream_t>(stream)>>>(
+          static_cast<const bf16_t *>(x), x_strides[0], static_cast<const bf16_t *>(weight),
+          w_stride_c, w_stride_k, static_cast<bf16_t *>(out), out_strides[0], seq_start, tokens,
+          channels, xb);
+    };
+    const bool w16 = wyh::aligned16(weight);
+    if (w_stride_c == 1 && w_stride_k % 8 == 0 && w16)
+      launch(seq_start ? conv4_prefill_vec_kernel<kConvVecRun, kTapRows, true>
+                       : conv4_prefill_vec_kernel<kConvVecRun, kTapRows, false>, kConvVecRun);
+    else if (w_stride_c == 4 && w_stride_k == 1 && w16)
+      launch(seq_start ? conv4_prefill_vec_kernel<kConvVecRun, kTapQuads, true>
+                       : conv4_prefill_vec_kernel<kConvVecRun, kTapQuads, false>, kConvVecRun);
+    else if (int64_t(xb) * tokens <= 512 * kConvVecRun)   // two workgroups to a CU
+      launch(seq_start ? conv4_prefill_vec_kernel<kConvVecRun, kTapAny, true>
+                       : conv4_prefill_vec_kernel<kConvVecRun, kTapAny, false>, kConvVecRun);
+    else
+      launch(seq_start ? conv4_prefill_vec_kernel<kConvRun, kTapAny, true>
+                       : conv4_prefill_vec_kernel<kConvRun, kTapAny, false>, kConvRun);
     return wyh::launch_status();
   }
   const dim3 grid(unsigned((channels + 255) / 256), runs);
