@@ -226,7 +226,7 @@ __global__ __launch_bounds__(64 * kNW) void gemm_skinny_kernel(
     for (int nt = 0; nt < kNT; ++nt) acc[mt][nt] = f32x4v_t{0.f, 0.f, 0.f, 0.f};
   // one 32-wide k-step of row tile mt; the A operand from what was loaded for it
   struct RawA {
-    u32x4_t x, r;   // x and the residual (kPro 1) or the up half (kPro 2)
+    u32x4_t x, r;   // x and the residual (kPro 1)
   };
   auto load_raw = [&](int mt, int kk) {
     RawA a;
@@ -234,8 +234,6 @@ __global__ __launch_bounds__(64 * kNW) void gemm_skinny_kernel(
     if constexpr (kPro == 1) {
       a.r = u32x4_t{0u, 0u, 0u, 0u};
       if (rp[mt]) a.r = ld16(rp[mt] + kk);
-    } else if constexpr (kPro == 2) {
-      a.r = ld16(xp[mt] + pro.up_off + kk);
     }
     return a;
   };
@@ -244,8 +242,6 @@ __global__ __launch_bounds__(64 * kNW) void gemm_skinny_kernel(
     if constexpr (kPro == 1) {
       if (rp[mt]) xv = add_bf16x8(xv, a.r);
       xv = norm_bf16x8(xv, rsr[mt], nw8);
-    } else if constexpr (kPro == 2) {
-      xv = swiglu_bf16x8(xv, a.r);
     }
     return xok[mt] ? xv : u32x4_t{0u, 0u, 0u, 0u};
   };
@@ -353,9 +349,55 @@ __global__ __launch_bounds__(64 * kNW) void gemm_skinny_kernel(
   };
   constexpr bool kOnce = kMT <= 2 && kNW <= 8;   // registers
   const bool fits = kPro != 1 || (K <= 1024 && M <= kOnceRows && rem == 0);
-  if (kOnce && fits && nfull == 1) {
+  if constexpr (kPro == 2) {
+    // Bound by the gate's VALU work, which a wave does as each pair of loads
+    // lands, the next pair in flight.  In the form below (all loads of a slice
+    // first, or padding rows' gates skipped by a branch, which keeps the next
+    // pair from being requested early) [1024, 3584] took 8.8 us at M = 16, 12.5
+    // at M = 32, 17.3 at M = 64; so 8.1, 10.4, 15.4.
+    const auto load_a = [&](int mt, int kk) {
+      return swiglu_bf16x8(ld16(xp[mt] + kk), ld16(xp[mt] + pro.up_off + kk));
+    };
+    const auto multiply = [&](auto steps, const u32x4_t (&wv)[decltype(steps)::value][kNT], int k) {
+      constexpr int R = decltype(steps)::value;
+      u32x4_t xv[kMT][R];
+#pragma unroll
+      for (int mt = 0; mt < kMT; ++mt)
+#pragma unroll
+        for (int j = 0; j < R; ++j) xv[mt][j] = load_a(mt, k + 32 * j);
+#pragma unroll
+      for (int j = 0; j < R; ++j)
+#pragma unroll
+        for (int mt = 0; mt < kMT; ++mt) {
+          if (!xok[mt]) xv[mt][j] = u32x4_t{0u, 0u, 0u, 0u};
+          step(acc, wv[j], xv[mt][j], mt);
+        }
+    };
+    const auto load_w = [&](auto &wv, int k) {
+#pragma unroll
+      for (int j = 0; j < int(sizeof(wv) / sizeof(wv[0])); ++j)
+#pragma unroll
+        for (int nt = 0; nt < kNT; ++nt) wv[j][nt] = ld16(wp[nt] + k + 32 * j);
+    };
+    const auto load_batch = [&](auto steps, int k) {
+      u32x4_t wv[decltype(steps)::value][kNT];
+      load_w(wv, k);
+      multiply(steps, wv, k);
+    };
+    using S4 = std::integral_constant<int, 4>;
+    u32x4_t w_first[4][kNT];
+    if (nfull > 0) {
+      load_w(w_first, 0);
+      multiply(S4{}, w_first, 0);
+    }
+    for (int b = 1; b < nfull; ++b) load_batch(S4{}, 128 * b);
+    const int kt = 128 * nfull;
+    if (rem == 1) load_batch(std::integral_constant<int, 1>{}, kt);
+    else if (rem == 2) load_batch(std::integral_constant<int, 2>{}, kt);
+    else if (rem == 3) load_batch(std::integral_constant<int, 3>{}, kt);
+  } else if (kOnce && fits && nfull == 1) {
     if (rem == 0) once(std::integral_constant<int, 4>{});
-    if constexpr (kPro != 1) {
+    if constexpr (kPro == 0) {
       if (rem == 1) once(std::integral_constant<int, 5>{});
       else if (rem == 2) once(std::integral_constant<int, 6>{});
       else if (rem == 3) once(std::integral_constant<int, 7>{});
@@ -414,7 +456,10 @@ __global__ __launch_bounds__(64 * kNW) void gemm_skinny_kernel(
         }
       }
     };
-    for (int b = 0; b < nfull; ++b) load_batch(std::integral_constant<int, 4>{}, 128 * b);
+    // (the first batch outside the loop: 2 to 4% at M = 33..64 where a wave has
+    // one batch or a few: [4096, 4096] at M = 64 27.1 us in it, 26.5 so)
+    if (nfull > 0) load_batch(std::integral_constant<int, 4>{}, 0);
+    for (int b = 1; b < nfull; ++b) load_batch(std::integral_constant<int, 4>{}, 128 * b);
     const int kt = 128 * nfull;
     if (rem == 1) load_batch(std::integral_constant<int, 1>{}, kt);
     else if (rem == 2) load_batch(std::integral_constant<int, 2>{}, kt);
