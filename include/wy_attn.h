@@ -509,6 +509,24 @@ int wy_gdn_prefill_varlen_max(const void *q, const int64_t *q_strides, const voi
                               int num_heads, int key_dim, int value_dim, float *workspace,
                               int64_t workspace_bytes, void *stream);
 
+/*
+ * wy_gdn_prefill_varlen for one prompt alone (state [1, H, key_dim,
+ * value_dim]), cut into segments of a length that suits its own, which differ
+ * from a packed batch's: the same values to the last bits of the fp32 sums.
+ * workspace: NULL / 0 bytes (no segments), or 16-byte aligned device memory of
+ * wy_gdn_prefill_prompt_workspace_bytes(T, H, value_dim) bytes.
+ * Replaces call_gdn_recurrent_prefill_chunked_triton
+ *   (triton_kernels/gdn_recurrent_prefill.py:1026-1048).
+ */
+int wy_gdn_prefill_prompt(const void *q, const int64_t *q_strides, const void *k,
+                          const int64_t *k_strides, const void *v, const int64_t *v_strides,
+                          const float *beta, const int64_t *beta_strides, const float *g,
+                          const int64_t *g_strides, void *out, const int64_t *out_strides,
+                          float *state, const int64_t *state_strides, int token_num,
+                          int num_heads, int key_dim, int value_dim, float *workspace,
+                          int64_t workspace_bytes, void *stream);
+int64_t wy_gdn_prefill_prompt_workspace_bytes(int token_num, int num_heads, int value_dim);
+
 /* Workspace size of wy_gdn_prefill_varlen (0: none needed). */
 int64_t wy_gdn_prefill_varlen_workspace_bytes(int token_num, int num_heads, int value_dim);
 

@@ -73,6 +73,8 @@ _SIGNATURES = {
     "wy_gdn_prefill_varlen_max": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp,
                               _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _i, _i, _i, _i, _i, _i, _vp,
                               _i64, _vp],
+    "wy_gdn_prefill_prompt": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp,
+                              _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _i, _i, _i, _i, _vp, _i64, _vp],
     "wy_depthwise_causal_conv4_decode": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp,
                                          _c_i64p, _i, _i, _vp],
     "wy_gdn_qk_norm_gates": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _vp,
@@ -98,6 +100,7 @@ _SIGNATURES = {
 _SIZE_QUERIES = ("wy_varlen_causal_prefill_workspace_bytes", "wy_gemm_2d_workspace_bytes",
                  "wy_gemm_2d_gate_up_swiglu_workspace_bytes",
                  "wy_lm_head_argmax_workspace_bytes", "wy_gdn_prefill_varlen_workspace_bytes",
+                 "wy_gdn_prefill_prompt_workspace_bytes",
                  "wy_paged_decode_step_noalloc_max_rows",
                  "wy_page_stream_read_waves")
 
@@ -131,7 +134,8 @@ def load() -> ctypes.CDLL:
     for fn in (lib.wy_varlen_causal_prefill_workspace_bytes, lib.wy_gemm_2d_workspace_bytes,
                lib.wy_gemm_2d_gate_up_swiglu_workspace_bytes,
                lib.wy_lm_head_argmax_workspace_bytes,
-               lib.wy_gdn_prefill_varlen_workspace_bytes):
+               lib.wy_gdn_prefill_varlen_workspace_bytes,
+               lib.wy_gdn_prefill_prompt_workspace_bytes):
         fn.argtypes = [_i, _i, _i]
         fn.restype = ctypes.c_int64
     for fn in (lib.wy_paged_decode_step_noalloc_max_rows, lib.wy_page_stream_read_waves):

@@ -28,13 +28,14 @@
 // four wavefronts and lie in LDS with that row order: token or key 4 hf + (i &
 // 3) + 8 (i >> 2) of a 16-group in slot 8 hf + i.
 //
-// Segments: a sequence longer than kSeg tokens is cut into segments that run
+// Segments: a sequence longer than seg_len tokens is cut into segments that run
 // side by side.  A first launch walks every segment but the last from a zero
 // state and, as 128 further columns with v = 0 from the identity, its
 // homogeneous solution P; a second folds S_{s+1} = P_s S_s + U_s along the
-// segments; the last launch walks all segments from their true states.  Where
-// a sequence is cut depends on its own length alone, so a sequence gives the
-// same bits in every batch.
+// segments; the last launch walks all segments from their true states.  In a
+// packed batch seg_len is kSeg, so that a sequence gives the same bits in every
+// batch; a prompt given as one alone has the chip to itself and takes the
+// length that suits it (prompt_segment).
 //
 // Values that are not finite (infinities and NaN in the inputs, sums past
 // FLT_MAX): the products spread them further than the recurrence does, and a
@@ -51,9 +52,7 @@
 // token): 32 x 128 tokens 200 -> 43 us, 24 prompts of 22..4096 tokens (23.8k)
 // 3.10 ms -> 0.47 ms, one prompt of 1000 tokens 304 -> 142 us, one of 5003
 // 287 (chunk ops of csrc/gdn_chunk.hip) -> 189 us; one of 9 to 16 tokens 6.4 to
-// 8.6 -> 9.5 us, the chunk's fixed cost.  Segment length (same cases, us; 128 / 256 / 512
-// / 1024 tokens): 23.8k mixed 710 / 557 / 470 / 402, 5003 250 / 194 / 189 /
-// 288, 1000 68 / 85 / 142 / 153.
+// 8.6 -> 9.5 us, the chunk's fixed cost.
 #include "gdn_common.h"
 
 using namespace wy;
@@ -63,10 +62,14 @@ namespace {
 
 constexpr int kC = 32;        // tokens per chunk
 constexpr int kG = 64;        // tokens staged together (two chunks)
+// Tokens per segment of a packed batch.  Shorter ones fill the chip when few
+// sequences are there, longer ones save walking twice what fills it anyway: 128
+// / 256 / 512 / 1024 tokens: 24 prompts of 22..4096 tokens 710 / 557 / 470 / 402
+// us, one of 5003 250 / 194 / 189 / 288, one of 1000 68 / 85 / 142 / 153.
 #ifndef WY_GDN_SEG
 #define WY_GDN_SEG 512
 #endif
-constexpr int kSeg = WY_GDN_SEG;   // tokens per segment
+constexpr int kSeg = WY_GDN_SEG;
 static_assert(kSeg % kG == 0, "segments hold whole groups");
 // Sequences of at most kWalk tokens are walked token by token: a chunk costs
 // the same whatever it holds.  One prompt, us a launch, walked by
@@ -235,19 +238,23 @@ __device__ __forceinline__ double lane_of(double x, int l) {
 __device__ __forceinline__ int seq_start(const int32_t *cu, int token_num, int i) {
   return cu ? cu[i] : i ? token_num : 0;
 }
-__device__ __forceinline__ int seg_count(int len) { return len > kSeg ? (len + kSeg - 1) / kSeg : 1; }
+__device__ __forceinline__ int seg_count(int len, int seg_len) {
+  return len > seg_len ? (len - 1) / seg_len + 1 : 1;
+}
 
 // Item `item` of the packed batch's segments (of all of them, or of all but
 // each sequence's last): its sequence, segment and the number of non-last
 // segments in the sequences before it (its workspace slots start there).
 // Each wavefront scans 64 sequences at a time.
-__device__ __forceinline__ bool find_segment(const int32_t *cu, int token_num, int batch, int item,
-                                             bool nonlast, int &b, int &s, int &slot0) {
+__device__ __forceinline__ bool find_segment(const int32_t *cu, int token_num, int batch, int seg_len,
+                                             int item, bool nonlast, int &b, int &s, int &slot0) {
   const int lane = threadIdx.x & 63;
   int items = 0, slots = 0;
   for (int b0 = 0; b0 < batch; b0 += 64) {
     const int i = b0 + lane;
-    const int n = i < batch ? seg_count(seq_start(cu, token_num, i + 1) - seq_start(cu, token_num, i)) : 0;
+    const int n =
+        i < batch ? seg_count(seq_start(cu, token_num, i + 1) - seq_start(cu, token_num, i), seg_len)
+                  : 0;
     const int extra = n > 0 ? n - 1 : 0, cnt = nonlast ? extra : n;
     int ci = cnt, si = extra;   // inclusive prefix sums
 #pragma unroll
@@ -273,11 +280,11 @@ __device__ __forceinline__ bool find_segment(const int32_t *cu, int token_num, i
 }
 
 // Non-last segments in the sequences before b (of a batch with cu_seqlens).
-__device__ __forceinline__ int slots_before(const int32_t *cu, int b, int lane) {
+__device__ __forceinline__ int slots_before(const int32_t *cu, int seg_len, int b, int lane) {
   int n = 0;
   for (int b0 = 0; b0 < b; b0 += 64) {
     const int i = b0 + lane;
-    int x = i < b ? seg_count(cu[i + 1] - cu[i]) - 1 : 0;
+    int x = i < b ? seg_count(cu[i + 1] - cu[i], seg_len) - 1 : 0;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
     n += x;
@@ -538,7 +545,7 @@ __device__ __forceinline__ void walk_not_finite(const GdnArgs &a, int s0, int t_
 // kState: a non-last segment's state (and homogeneous solution) only.
 template <bool kContig, bool kState>
 __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int token_num, int batch,
-                                                          float *ws, int slots) {
+                                                          float *ws, int slots, int seg_len) {
   extern __shared__ __align__(16) unsigned char scan_smem[];
   ScanLds &L = *reinterpret_cast<ScanLds *>(scan_smem);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -563,8 +570,8 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
     if (b >= batch) return;
   } else if (listed) {
     b = item - slots;
-  } else if (!find_segment(a.cu_seqlens, token_num, batch, item, kState || batch > 64, b, seg,
-                           slot0)) {
+  } else if (!find_segment(a.cu_seqlens, token_num, batch, seg_len, item, kState || batch > 64,
+                           b, seg, slot0)) {
     return;
   }
   // the same in every lane: pointers and buffer resources built from them
@@ -580,15 +587,15 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
       return;
     }
   }
-  const int nseg = slots == 0 ? 1 : seg_count(len);
+  const int nseg = slots == 0 ? 1 : seg_count(len, seg_len);
   if (listed && nseg > 1) {
     seg = nseg - 1;
-    slot0 = slots_before(a.cu_seqlens, b, lane);
+    slot0 = slots_before(a.cu_seqlens, seg_len, b, lane);
   }
   if (slot0 + nseg - 1 > slots) return;   // more tokens than the workspace was sized for
   if (hom && seg == 0) return;            // the first segment starts from a known (zero) state
-  const int t_lo = slots == 0 ? 0 : seg * kSeg;
-  const int t_hi = slots == 0 ? len : min(len, t_lo + kSeg);
+  const int t_lo = slots == 0 ? 0 : seg * seg_len;
+  const int t_hi = slots == 0 ? len : min(len, t_lo + seg_len);
   const int col = (hom ? 0 : vb * 128) + wave * kWCols + lr;
 
   // Where the state goes, and the distance of its rows: formed here, not by
@@ -1102,16 +1109,17 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
 // place of U_s.  Workgroup = one (sequence, head, 32 value columns); wave w
 // forms rows 32 w .. + 31, the cut state goes through LDS in operand order.
 __global__ __launch_bounds__(256) void gdn_fold_kernel(const int32_t *cu, int token_num, int heads,
-                                                       int dv, float *ws, int slots) {
+                                                       int dv, float *ws, int slots, int seg_len) {
   __shared__ __align__(16) u32x4_t sp[2][8][3][64];   // k-step, piece, lane; two steps' worth
   const int h = blockIdx.x % heads;
   const int cb = (blockIdx.x / heads) % (dv / kWCols);
   const int b = blockIdx.x / (heads * (dv / kWCols));
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lr = lane & 31, hf = lane >> 5;
-  const int nseg = seg_count(seq_start(cu, token_num, b + 1) - seq_start(cu, token_num, b));
+  const int nseg =
+      seg_count(seq_start(cu, token_num, b + 1) - seq_start(cu, token_num, b), seg_len);
   if (nseg < 3) return;   // S_1 = U_0 needs no fold
-  const int slot0 = slots_before(cu, b, lane);   // (b > 0: there is a cu)
+  const int slot0 = slots_before(cu, seg_len, b, lane);   // (b > 0: there is a cu)
   if (slot0 + nseg - 1 > slots) return;
   const int col = cb * kWCols + lr;
   const int row0 = 32 * wave + 4 * hf;
@@ -1191,7 +1199,8 @@ int launch_walk(const GdnArgs &a, int token_num, int batch, hipStream_t st) {
 }
 
 template <bool kContig>
-int launch_scan(const GdnArgs &a, int token_num, int batch, float *ws, int slots, hipStream_t st) {
+int launch_scan(const GdnArgs &a, int token_num, int batch, float *ws, int slots, int seg_len,
+                hipStream_t st) {
   const int vblocks = a.dv / 128;
   const int64_t main = int64_t(batch + slots) * a.heads * vblocks;
   const int64_t pre = int64_t(slots) * a.heads * (vblocks + 1);
@@ -1209,11 +1218,12 @@ int launch_scan(const GdnArgs &a, int token_num, int batch, float *ws, int slots
   if (rc1 != hipSuccess) return int(rc1);
   if (slots > 0) {
     gdn_scan_kernel<kContig, true>
-        <<<unsigned(pre), 256, sizeof(ScanLds), st>>>(a, token_num, batch, ws, slots);
-    gdn_fold_kernel<<<unsigned(fold), 256, 0, st>>>(a.cu_seqlens, token_num, a.heads, a.dv, ws, slots);
+        <<<unsigned(pre), 256, sizeof(ScanLds), st>>>(a, token_num, batch, ws, slots, seg_len);
+    gdn_fold_kernel<<<unsigned(fold), 256, 0, st>>>(a.cu_seqlens, token_num, a.heads, a.dv, ws,
+                                                    slots, seg_len);
   }
   gdn_scan_kernel<kContig, false>
-      <<<unsigned(main), 256, sizeof(ScanLds), st>>>(a, token_num, batch, ws, slots);
+      <<<unsigned(main), 256, sizeof(ScanLds), st>>>(a, token_num, batch, ws, slots, seg_len);
   return wyh::launch_status();
 }
 
@@ -1221,12 +1231,57 @@ int launch_scan(const GdnArgs &a, int token_num, int batch, float *ws, int slots
 // whole kSeg tokens.
 int64_t slot_bound(int64_t token_num) { return token_num > kSeg ? token_num / kSeg : 0; }
 
+// Segment length of one prompt alone: the two walks grow with it, the fold with
+// their number.  us by segment length 64 / 128 / 192 / 256 / 384 / 512 (16
+// heads; before them the chunk ops of csrc/gdn_chunk.hip): 257 tokens 44: 43 /
+// 50 / 59 / 75 / 49 / 49; 512 53: 56 / 56 / 68 / 79 / 107 / 80; 1000 70: 90 /
+// 75 / 82 / 90 / 117 / 145; 2048 115: 170 / 115 / 112 / 110 / 133 / 156; 3000
+// 168: 245 / 165 / 134 / 137 / 143 / 165; 5003 274: 403 / 269 / 213 / 208 / 182
+// / 205; 8192 474: 675 / 405 / 337 / 275 / 269 / 237.
+int prompt_segment(int token_num) {
+  if (token_num <= 192) return 192;   // 130 tokens: 30 in one piece, 34 in three
+  const int len = (token_num / 16 + 64 + kG / 2) / kG * kG;
+  return len < kSeg ? len : kSeg;
+}
+int64_t prompt_slots(int token_num) {
+  return token_num > 0 ? (token_num - 1) / prompt_segment(token_num) : 0;
+}
+int64_t slots_bytes(int64_t slots, int heads, int dv) {
+  return slots * heads * kDK * (int64_t(dv) + kDK) * 4;
+}
+
 }  // namespace
 
 extern "C" int64_t wy_gdn_prefill_varlen_workspace_bytes(int token_num, int num_heads,
                                                          int value_dim) {
   if (token_num <= 0 || num_heads <= 0 || value_dim <= 0) return 0;
-  return slot_bound(token_num) * num_heads * kDK * (int64_t(value_dim) + kDK) * 4;
+  return slots_bytes(slot_bound(token_num), num_heads, value_dim);
+}
+
+extern "C" int64_t wy_gdn_prefill_prompt_workspace_bytes(int token_num, int num_heads,
+                                                         int value_dim) {
+  if (token_num <= 0 || num_heads <= 0 || value_dim <= 0) return 0;
+  return slots_bytes(prompt_slots(token_num), num_heads, value_dim);
+}
+
+// slots: segments that the workspace holds (0: none are cut)
+static int run_prefill(GdnArgs &a, bool contig, int token_num, int max_seqlen, int batch,
+                       float *workspace, int64_t workspace_bytes, int64_t slots, int seg_len,
+                       hipStream_t st) {
+  const int bound = max_seqlen > 0 ? max_seqlen : token_num;   // 0: unknown
+  if (bound > 0 && bound <= kWalk && batch <= kWalkBatch)
+    return contig ? launch_walk<true>(a, token_num, batch, st)
+                  : launch_walk<false>(a, token_num, batch, st);
+  if (slots > 0x7fffffff / 2) return WY_E_SHAPE;
+  if (slots > 0 && workspace_bytes < slots_bytes(slots, a.heads, a.dv)) return WY_E_CAPACITY;
+  if (slots > 0 && !wyh::aligned16(workspace)) return WY_E_LAYOUT;
+  // the buffer-resource form: rows at least as long as what is read of them,
+  // and a group of them within 31 bits of bytes
+  const auto row_ok = [](int64_t t, int64_t width) { return t >= width && t < (1 << 22); };
+  contig = contig && row_ok(a.q_t, kDK) && row_ok(a.k_t, kDK) && row_ok(a.v_t, a.dv) &&
+           row_ok(a.o_t, a.dv) && row_ok(a.s_k, a.dv) && row_ok(a.g_t, 1) && row_ok(a.beta_t, 1);
+  return contig ? launch_scan<true>(a, token_num, batch, workspace, int(slots), seg_len, st)
+                : launch_scan<false>(a, token_num, batch, workspace, int(slots), seg_len, st);
 }
 
 extern "C" int wy_gdn_prefill_varlen_max(
@@ -1246,24 +1301,30 @@ extern "C" int wy_gdn_prefill_varlen_max(
   if (batch < 0 || token_num < 0 || max_seqlen < 0) return WY_E_SHAPE;
   if (batch == 0) return WY_OK;
   a.cu_seqlens = cu_seqlens;
-  const hipStream_t st = static_cast<hipStream_t>(stream);
-  const int bound = max_seqlen > 0 ? max_seqlen : token_num;   // 0: unknown
-  if (bound > 0 && bound <= kWalk && batch <= kWalkBatch)
-    return contig ? launch_walk<true>(a, token_num, batch, st)
-                  : launch_walk<false>(a, token_num, batch, st);
-  const int64_t slots = workspace ? slot_bound(token_num) : 0;
-  if (slots > 0x7fffffff / 2) return WY_E_SHAPE;
-  if (slots > 0 && workspace_bytes <
-                       wy_gdn_prefill_varlen_workspace_bytes(token_num, num_heads, value_dim))
-    return WY_E_CAPACITY;
-  if (slots > 0 && !wyh::aligned16(workspace)) return WY_E_LAYOUT;
-  // the buffer-resource form: rows at least as long as what is read of them,
-  // and a group of them within 31 bits of bytes
-  const auto row_ok = [](int64_t t, int64_t width) { return t >= width && t < (1 << 22); };
-  contig = contig && row_ok(a.q_t, kDK) && row_ok(a.k_t, kDK) && row_ok(a.v_t, a.dv) &&
-           row_ok(a.o_t, a.dv) && row_ok(a.s_k, a.dv) && row_ok(a.g_t, 1) && row_ok(a.beta_t, 1);
-  return contig ? launch_scan<true>(a, token_num, batch, workspace, int(slots), st)
-                : launch_scan<false>(a, token_num, batch, workspace, int(slots), st);
+  return run_prefill(a, contig, token_num, max_seqlen, batch, workspace, workspace_bytes,
+                     workspace ? slot_bound(token_num) : 0, kSeg,
+                     static_cast<hipStream_t>(stream));
+}
+
+extern "C" int wy_gdn_prefill_prompt(const void *q, const int64_t *q_strides, const void *k,
+                                     const int64_t *k_strides, const void *v,
+                                     const int64_t *v_strides, const float *beta,
+                                     const int64_t *beta_strides, const float *g,
+                                     const int64_t *g_strides, void *out,
+                                     const int64_t *out_strides, float *state,
+                                     const int64_t *state_strides, int token_num, int num_heads,
+                                     int key_dim, int value_dim, float *workspace,
+                                     int64_t workspace_bytes, void *stream) {
+  GdnArgs a;
+  bool contig = false;
+  const int rc = gdn_setup(a, contig, q, q_strides, k, k_strides, v, v_strides, beta,
+                           beta_strides, g, g_strides, out, out_strides, state, state_strides,
+                           num_heads, key_dim, value_dim);
+  if (rc != WY_OK) return rc;
+  if (token_num <= 0) return WY_E_SHAPE;
+  return run_prefill(a, contig, token_num, token_num, 1, workspace, workspace_bytes,
+                     workspace ? prompt_slots(token_num) : 0, prompt_segment(token_num),
+                     static_cast<hipStream_t>(stream));
 }
 
 extern "C" int wy_gdn_prefill_varlen(const void *q, const int64_t *q_strides, const void *k,

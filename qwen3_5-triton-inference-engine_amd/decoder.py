@@ -35,7 +35,7 @@ from .depthwise_causal_conv4_prefill import depthwise_causal_conv4_prefill
 from .gdn_gated_rmsnorm import gdn_gated_rmsnorm
 from .gdn_qk_norm_gates import gdn_qk_norm_gates
 from .gdn_recurrent_prefill import (
-    call_gdn_recurrent_prefill_chunked_triton,
+    gdn_prefill_prompt_into,
     gdn_prefill_sequential_into,
 )
 
@@ -319,10 +319,9 @@ class DecodeModel:
                                             fused[:, 4 * HD + H:], w.extra["a_log"],
                                             w.extra["dt_bias"])
         if packed.batch == 1 and T >= GDN_CHUNKED_PREFILL_MIN_TOKENS:
-            # one long prompt: the chunk-64 WY path (engine/runner.py:272-273)
-            core, state = call_gdn_recurrent_prefill_chunked_triton(qn, kn, v, beta, g)
-            state = state.unsqueeze(0)
-            self.rec_states[i].copy_(state)
+            # one long prompt: segments of a length that suits it (the reference's
+            # chunked route, engine/runner.py:272-273)
+            core = gdn_prefill_prompt_into(qn, kn, v, beta, g, self.rec_states[i])
         else:
             core = gdn_prefill_sequential_into(qn, kn, v, beta, g, packed.cu_seqlens,
                                                self.rec_states[i], packed.max_seqlen)

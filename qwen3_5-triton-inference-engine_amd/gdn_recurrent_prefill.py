@@ -312,8 +312,46 @@ def call_gdn_chunk_output_triton(q, k, delta, g_cumsum, chunk_state):
     return gdn_chunk_output(q, k, delta, g_cumsum, chunk_state)
 
 
+def gdn_prefill_prompt_into(q, k, v, beta, g, state):
+    """One prompt through the segment kernels, its final state into ``state``
+    (``[1, H, DK, DV]`` fp32).  Returns ``out [T, H, DV]`` bf16."""
+    _check_common(q, k, v, beta, g)
+    token_num, num_heads, key_dim = q.shape
+    value_dim = v.shape[-1]
+    assert token_num > 0 and num_heads > 0
+    assert state.dtype == torch.float32
+    assert state.shape == (1, num_heads, key_dim, value_dim)
+    out = torch.empty_like(v)
+    nbytes = _lib.load().wy_gdn_prefill_prompt_workspace_bytes(token_num, num_heads, value_dim)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+    _lib.call(
+        "wy_gdn_prefill_prompt", *_tensor_args(q, k, v, beta, g, out, state), token_num,
+        num_heads, key_dim, value_dim, _lib.ptr(ws), nbytes, _lib.stream(q.device),
+    )
+    return out
+
+
+@torch.library.custom_op("wy_lib::gdn_prefill_prompt", mutates_args=(), device_types="cuda")
+def gdn_prefill_prompt(
+    q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: torch.Tensor, g: torch.Tensor
+) -> tuple[torch.Tensor, torch.Tensor]:
+    """One prompt alone: ``(out [T, H, DV] bf16, final_state [H, DK, DV] fp32)``.
+    The recurrence of ``gdn_recurrent_prefill_sequential``, cut into segments of
+    a length chosen for this prompt (there one length for every batch)."""
+    state = torch.empty((1, q.shape[1], q.shape[2], v.shape[-1]), dtype=torch.float32,
+                        device=q.device)
+    out = gdn_prefill_prompt_into(q, k, v, beta, g, state)
+    return out, state[0]
+
+
+@gdn_prefill_prompt.register_fake
+def _gdn_prefill_prompt_fake(q, k, v, beta, g):
+    return torch.empty_like(v), torch.empty((q.shape[1], q.shape[2], v.shape[2]),
+                                            dtype=torch.float32, device=q.device)
+
+
 def call_gdn_recurrent_prefill_chunked_triton(q, k, v, beta, g):
     """One prompt: ``(out [T, H, DV] bf16, final_state [H, DK, DV] fp32)``, the
     result of the chunk ops above (reference gdn_recurrent_prefill.py:1026-1048)
     by the packed prefill's kernels, which form no intermediate tensors."""
-    return gdn_recurrent_prefill_sequential(q, k, v, beta, g)
+    return gdn_prefill_prompt(q, k, v, beta, g)

@@ -101,6 +101,19 @@ def test_short_sequences_same_bits_by_every_route(pkg, dev, lens):
     assert rel(out[rows], o64) < 2 ** -9 and rel(st[some], s64) < 1e-6
 
 
+# one prompt alone: walked, in one piece, at the first cut, a segment's edges
+@pytest.mark.parametrize("T", [1, 8, 9, 64, 192, 193, 256, 257, 1024, 1025, 2100])
+def test_prompt_alone_vs_recurrence(pkg, dev, T):
+    args = inputs(T, dev, 23 + T, 0.003)
+    out, st = pkg.call_gdn_recurrent_prefill_chunked_triton(*args)
+    o64, s64 = recurrence64(*args, [T])
+    assert out.shape == (T, H, D) and st.shape == (H, D, D)
+    assert rel(out, o64) < 2 ** -9 and rel(st, s64[0]) < 1e-6
+    state = torch.full((1, H, D, D), float("nan"), device=dev)
+    got = pkg.gdn_recurrent_prefill.gdn_prefill_prompt_into(*args, state)
+    assert torch.equal(got, out) and torch.equal(state[0], st)
+
+
 @pytest.mark.parametrize("T", [7, 33, SEG + 70])
 def test_other_strides_same_bits(pkg, dev, T):
     q, k, v, beta, g = inputs(T, dev, T)
