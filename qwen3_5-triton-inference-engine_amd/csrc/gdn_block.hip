@@ -51,8 +51,15 @@ __device__ __forceinline__ uint32_t conv4_silu(float s1, float s2, float s3, flo
 // wavefronts (waves 2r, 2r+1): xor butterfly in each wave, then wave 2r's
 // part + wave 2r+1's part.  Every thread of the block must call it (it holds
 // a barrier); part needs one float per wave.
+// kLds: the exchanges through the LDS (same pairs, same bits).
+template <bool kLds = false>
 __device__ __forceinline__ float sum128(float v, float *part) {
-  v = wave_sum(v);
+  if constexpr (kLds) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  } else {
+    v = wave_sum(v);
+  }
   const int wave = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) part[wave] = v;
   __syncthreads();
@@ -469,6 +476,13 @@ struct BlockArgs {
 //   2. waves 0-1 / 2-3: q / k L2 norm (sum128, as the standalone kernel);
 //   3. every wave: one recurrence step on its 16 value columns (gdn_step);
 //   4. waves 0-1: gated RMSNorm of the bf16 step output with z.
+// kMany: more workgroups than the chip holds at once.  Then the memory is the
+// bound, and the norms' sums stay LDS permutes: with the shorter VALU chains a
+// workgroup's stores come sooner after its loads, in the way of the next one's
+// (us, LDS / VALU: 16 sequences 9.2 / 9.1, 24 13.7 / 13.1, 32 14.7 / 14.2, 40
+// 20.3 / 21.2, 48 22.1 / 24.2, 64 28.8 / 29.7, 128 54.6 / 56.7, 256 110.8 / 114.3).
+constexpr int kChipBlocks = 512;   // two 512-thread workgroups to each of 256 CUs
+template <bool kMany>
 __global__ __launch_bounds__(512) void gdn_decode_block_kernel(const BlockArgs p) {
   __shared__ float y_lds[3 * kDK];  // conv outputs (bf16 values): q | k | v
   __shared__ float qk_lds[2 * kDK]; // normalised q | k (bf16 values)
@@ -521,7 +535,7 @@ __global__ __launch_bounds__(512) void gdn_decode_block_kernel(const BlockArgs p
   // 2. q / k L2 norm: waves 0-1 hold q, waves 2-3 k (threads 256.. add zeros)
   {
     const float x = tid < 2 * kDK ? y_lds[tid] : 0.f;
-    const float ss = sum128(x * x, part);
+    const float ss = sum128<kMany>(x * x, part);
     const float r = rsqrtf(ss + 1e-6f);
     if (tid < kDK)
       qk_lds[tid] = bf16_to_f32(bf16_t(f32_to_bf16_bits((x * r) * p.q_scale)));
@@ -555,7 +569,7 @@ __global__ __launch_bounds__(512) void gdn_decode_block_kernel(const BlockArgs p
   // 4. gated RMSNorm (waves 0-1; the others add zeros to their own pairs)
   {
     const float x = tid < kDK ? core[tid] : 0.f;
-    const float ss = sum128(x * x, part + 0);
+    const float ss = sum128<kMany>(x * x, part + 0);
     if (tid < kDK) {
       const float inv = rsqrtf(ss / float(kDK) + 1e-6f);
       p.out[b * p.o_b + h * kDK + tid] =
@@ -691,8 +705,11 @@ extern "C" int wy_gdn_decode_block(const void *fused, int64_t fused_stride0, voi
   p.o_b = out_stride0;
   p.heads = num_heads;
   p.q_scale = float(1.0 / sqrt(double(head_dim)));
-  gdn_decode_block_kernel<<<unsigned(batch * num_heads), 512, 0,
-                            static_cast<hipStream_t>(stream)>>>(p);
+  const unsigned blocks = unsigned(batch * num_heads);
+  if (blocks > kChipBlocks)
+    gdn_decode_block_kernel<true><<<blocks, 512, 0, static_cast<hipStream_t>(stream)>>>(p);
+  else
+    gdn_decode_block_kernel<false><<<blocks, 512, 0, static_cast<hipStream_t>(stream)>>>(p);
   return wyh::launch_status();
 }
 
