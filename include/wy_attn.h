@@ -258,6 +258,13 @@ void wy_prefill_set_ticket_order(int order);
 void wy_prefill_set_short_path(int enable);
 
 /*
+ * Test hook, no counterpart in the reference: adds to *mismatches (device) how
+ * many floats with the bits first .. last have a short reciprocal (the prompt
+ * conv's SiLU) that is not the division's bit for bit.
+ */
+int wy_check_short_reciprocal(uint32_t first, uint32_t last, int32_t *mismatches, void *stream);
+
+/*
  * Prefill attention block: the reference's prefill attention sequence after
  * the q/k RMSNorm (engine/runner.py:336-384) in two launches, bit-identical
  * to it.  Replaces, in order:

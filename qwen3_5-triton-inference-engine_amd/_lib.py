@@ -73,6 +73,7 @@ _SIGNATURES = {
     "wy_gdn_prefill_varlen_max": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp,
                               _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _i, _i, _i, _i, _i, _i, _vp,
                               _i64, _vp],
+    "wy_check_short_reciprocal": [ctypes.c_uint32, ctypes.c_uint32, _vp, _vp],
     "wy_gdn_prefill_prompt": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp,
                               _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _i, _i, _i, _i, _vp, _i64, _vp],
     "wy_depthwise_causal_conv4_decode": [_vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, _vp,

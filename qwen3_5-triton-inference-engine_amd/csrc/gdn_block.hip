@@ -32,7 +32,8 @@ __device__ __forceinline__ float conv4_silu_f(float s1, float s2, float s3, floa
   return acc * (1.0f / (1.0f + __expf(-acc)));
 }
 // The bits of the division 1 / d for 1 <= d <= 2^126 (and NaN for NaN): one
-// Newton step on v_rcp_f32, compared with the division for every such float.
+// Newton step on v_rcp_f32.  (wy_check_short_reciprocal compares it with the
+// division for every such float.)
 __device__ __forceinline__ float recip_ranged(float d) {
   const float r = __builtin_amdgcn_rcpf(d);
   return __fmaf_rn(__fmaf_rn(-d, r, 1.0f), r, r);
@@ -168,6 +169,18 @@ __global__ __launch_bounds__(128) void gdn_gated_rmsnorm_kernel(
 // for bit on the same window.
 constexpr int kConvRun = 16;
 constexpr int kConvVecRun = 4;  // the vectorised kernel's, measured there
+// Floats with the bits first .. last whose short reciprocal is not the division's.
+__global__ __launch_bounds__(256) void check_reciprocal_kernel(uint32_t first, uint32_t last,
+                                                               int32_t *mismatches) {
+  int n = 0;
+  const uint64_t step = uint64_t(gridDim.x) * 256;
+  for (uint64_t u = uint64_t(first) + blockIdx.x * 256 + threadIdx.x; u <= last; u += step) {
+    const float d = __uint_as_float(uint32_t(u));
+    n += __float_as_uint(recip_ranged(d)) != __float_as_uint(1.0f / d);
+  }
+  if (n) atomicAdd(mismatches, n);
+}
+
 // Row counts from which the norm ops take the row-vectorised kernels (the
 // decode sizes keep one block per row, the same reduction either way).
 constexpr int kVecRows = 256;
@@ -753,6 +766,15 @@ extern "C" int wy_depthwise_causal_conv4_prefill(const void *x, const int64_t *x
       static_cast<const bf16_t *>(x), x_strides[0], x_strides[1],
       static_cast<const bf16_t *>(weight), w_stride_c, w_stride_k, static_cast<bf16_t *>(out),
       out_strides[0], out_strides[1], seq_start, tokens, channels);
+  return wyh::launch_status();
+}
+
+extern "C" int wy_check_short_reciprocal(uint32_t first, uint32_t last, int32_t *mismatches,
+                                         void *stream) {
+  if (!mismatches) return WY_E_NULL;
+  if (first > last) return WY_E_SHAPE;
+  check_reciprocal_kernel<<<2048, 256, 0, static_cast<hipStream_t>(stream)>>>(first, last,
+                                                                              mismatches);
   return wyh::launch_status();
 }
 

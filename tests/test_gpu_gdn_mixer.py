@@ -252,3 +252,50 @@ def test_qk_norm_gates_last_block(pkg, dev, rows):
     got = pkg.gdn_qk_norm_gates(*(t.to(dev) for t in (q, k, a, b, a_log, dt)))
     for x, ref in zip(got, go.gdn_qk_norm_gates(q, k, a, b, a_log, dt)):
         close(x, ref)
+
+
+@pytest.mark.parametrize("T, Cs", [(1, 8), (33, 2056), (680, 6144), (690, 6144), (2050, 1000)])
+def test_conv4_prefill_weight_strides_same_bits(pkg, dev, T, Cs):
+    """Weights as [C, 4] rows in 16-byte loads, the same rows off their
+    alignment, apart, and as rows of channels; both sides of the number of runs
+    from which weights of any strides share their loads over longer ones."""
+    say(f"conv4 prefill weight strides T={T} C={Cs}")
+    gen = torch.Generator().manual_seed(T)
+    x = torch.randn(T, Cs, generator=gen).to(torch.bfloat16).to(dev)
+    w = torch.randn(Cs, 4, generator=gen).to(torch.bfloat16).to(dev)
+    off = torch.empty(Cs * 4 + 1, dtype=torch.bfloat16, device=dev)[1:].view(Cs, 4)
+    apart = torch.empty(Cs, 12, dtype=torch.bfloat16, device=dev)[:, ::3]
+    starts = (torch.arange(T, dtype=torch.int32) // 7 * 7).to(dev)
+    for s in (None, starts):
+        ref = pkg.depthwise_causal_conv4_prefill(x, w.t().contiguous().t(), s)
+        for wt in (w, off, apart):
+            wt.copy_(w)
+            assert torch.equal(pkg.depthwise_causal_conv4_prefill(x, wt, s), ref)
+
+
+@pytest.mark.parametrize("B", [33, 70])
+def test_decode_block_same_bits_past_a_full_chip(pkg, dev, B):
+    """Batches that fill the chip more than once take the other reduction."""
+    say(f"gdn decode block B={B} in parts")
+    fused, cs, cw, al, dt, nw, st = (x.to(dev) for x in mixer_inputs(B, 77))
+    parts = []
+    for lo in range(0, B, 32):
+        hi = min(lo + 32, B)
+        c, s = cs[lo:hi].clone(), st[lo:hi].clone()
+        parts.append((pkg.gdn_decode_block(fused[lo:hi], c, cw, al, dt, nw, s), c, s))
+    out = pkg.gdn_decode_block(fused, cs, cw, al, dt, nw, st)
+    for whole, i in ((out, 0), (cs, 1), (st, 2)):
+        assert torch.equal(whole, torch.cat([p[i] for p in parts]))
+
+
+def test_short_reciprocal_is_the_division(pkg, dev):
+    """Every float from 1 to 2^126, bit for bit."""
+    say("short reciprocal")
+    n = torch.zeros(1, dtype=torch.int32, device=dev)
+    one, top = 0x3f800000, (126 + 127) << 23
+    pkg._lib.call("wy_check_short_reciprocal", one, top, pkg._lib.ptr(n), pkg._lib.stream(dev))
+    assert int(n) == 0
+    # (past the range it is not: the comparison does count)
+    pkg._lib.call("wy_check_short_reciprocal", top, 0x7f800000, pkg._lib.ptr(n),
+                  pkg._lib.stream(dev))
+    assert int(n) > 0
