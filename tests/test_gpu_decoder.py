@@ -236,12 +236,24 @@ def test_prefill_then_decode_equals_token_by_token_decode(pkg, dev):
         b.pos.add_(1)
 
 
-def test_long_prompt_prefill_chunked_equals_sequential(pkg, dev, monkeypatch):
-    """One 2100-token prompt takes the chunk-64 GDN prefill (engine/runner.py:
-    272-273); the same prompt with the routing threshold raised takes the
-    sequential kernel: the recurrent and conv states, the K/V pages and the
-    next decode step agree within the kernels' rounding."""
-    say("decoder long-prompt prefill: chunked vs sequential GDN")
+def chunk_ops_into(pkg):
+    def run(q, k, v, beta, g, state):
+        w, u, G = pkg.gdn_chunk_prepare_wy(k, v, beta, g)
+        delta, cs, final = pkg.gdn_chunk_state(k, w, u, G)
+        state[0].copy_(final)
+        return pkg.gdn_chunk_output(q, k, delta, G, cs)
+    return run
+
+
+@pytest.mark.parametrize("other", ["packed", "chunk ops"])
+def test_long_prompt_prefill_chunked_equals_sequential(pkg, dev, monkeypatch, other):
+    """One 2100-token prompt takes the GDN prefill of a prompt alone (the
+    reference's chunked route, engine/runner.py:272-273); the same prompt with
+    the routing threshold raised takes the packed batches' segments, with the
+    chunk-64 ops in its place another algorithm: the recurrent and conv states,
+    the K/V pages and the next decode step agree within the kernels'
+    rounding."""
+    say(f"decoder long-prompt prefill: prompt alone vs {other}")
     import qwen35_amd.decoder as dmod
     cfg = tiny_cfg(pkg, layers=4)
     L = 2100
@@ -251,7 +263,10 @@ def test_long_prompt_prefill_chunked_equals_sequential(pkg, dev, monkeypatch):
     b = build(pkg, dev, cfg, 1, L + 8, True, seed=31)
     assert dmod.GDN_CHUNKED_PREFILL_MIN_TOKENS <= L
     ta = a.prefill(prompt, [L])
-    monkeypatch.setattr(dmod, "GDN_CHUNKED_PREFILL_MIN_TOKENS", L + 1)
+    if other == "packed":
+        monkeypatch.setattr(dmod, "GDN_CHUNKED_PREFILL_MIN_TOKENS", L + 1)
+    else:
+        monkeypatch.setattr(dmod, "gdn_prefill_prompt_into", chunk_ops_into(pkg))
     tb = b.prefill(prompt, [L])
     torch.cuda.synchronize()
     # the first GDN layer sees identical inputs: the kernels' own bound; later

@@ -1,7 +1,8 @@
 """GPU parity of the Gated DeltaNet chunk-64 (WY) prefill ops
 (wy_lib::gdn_chunk_prepare_wy / gdn_chunk_state / gdn_chunk_output and
 their chain) against the CPU oracle: each stage against the oracle's stage
-on the same inputs (fp64 there; bounds below), and the chain against the
+on the same inputs (fp64 there; bounds below), and the chain of the three ops
+as well as the wrapper (which runs the packed prefill's kernels) against the
 sequential recurrence at the reference's own bounds (out atol/rtol 1e-2,
 final state 2e-4) and against this build's sequential kernel.  The oracle's
 chunked form is pinned to the sequential one in tests/test_oracle_gdn.py."""
@@ -27,6 +28,18 @@ def inputs(T, seed, heads=H):
     return go.make_gdn_inputs(T, heads, DK, DV, torch.Generator().manual_seed(seed))
 
 
+def chain(pkg, q, k, v, beta, g):
+    """The three chunk ops, each on the one before."""
+    w, u, G = pkg.gdn_chunk_prepare_wy(k, v, beta, g)
+    delta, cs, final = pkg.gdn_chunk_state(k, w, u, G)
+    return pkg.gdn_chunk_output(q, k, delta, G, cs), final
+
+
+def form(pkg, which):
+    return {"chain": lambda *a: chain(pkg, *a),
+            "wrapper": pkg.call_gdn_recurrent_prefill_chunked_triton}[which]
+
+
 @pytest.mark.parametrize("T", [1, 63, 64, 65, 200])
 def test_chunk_stages_vs_oracle(pkg, dev, T):
     say(f"gdn chunk stages T={T}")
@@ -49,15 +62,16 @@ def test_chunk_stages_vs_oracle(pkg, dev, T):
     torch.testing.assert_close(out.float().cpu().double(), o_r, atol=1e-2, rtol=1e-2)
 
 
+@pytest.mark.parametrize("which", ["chain", "wrapper"])
 @pytest.mark.parametrize("T", [300, 2048, 4096])
-def test_chunked_prefill_vs_sequential(pkg, dev, T):
-    """The chain against the sequential recurrence (oracle and this build's
-    sequential kernel); T = 4096 is the single long prompt the runner sends
-    down the chunked path (engine/runner.py:151-153, 272)."""
+def test_chunked_prefill_vs_sequential(pkg, dev, T, which):
+    """Chain and wrapper against the sequential recurrence (oracle and this
+    build's sequential kernel); T = 4096 is the single long prompt the runner
+    sends down the chunked path (engine/runner.py:151-153, 272)."""
     say(f"gdn chunked prefill T={T}")
     q, k, v, beta, g = inputs(T, T)
     qd, kd, vd, bd, gd = (x.to(dev) for x in (q, k, v, beta, g))
-    out, st = pkg.call_gdn_recurrent_prefill_chunked_triton(qd, kd, vd, bd, gd)
+    out, st = form(pkg, which)(qd, kd, vd, bd, gd)
     torch.cuda.synchronize()
     assert out.shape == (T, H, DV) and st.shape == (H, DK, DV)
     o_seq, s_seq = pkg.gdn_recurrent_prefill_sequential(qd, kd, vd, bd, gd)
@@ -70,7 +84,8 @@ def test_chunked_prefill_vs_sequential(pkg, dev, T):
     torch.testing.assert_close(st.cpu(), s_r[0], atol=2e-4, rtol=2e-4)
 
 
-def test_chunked_prefill_strided_inputs(pkg, dev):
+@pytest.mark.parametrize("which", ["chain", "wrapper"])
+def test_chunked_prefill_strided_inputs(pkg, dev, which):
     """q, k, v as column slices of wider rows (the runner's views of the conv
     output): same result as contiguous copies."""
     say("gdn chunked prefill strided inputs")
@@ -79,7 +94,7 @@ def test_chunked_prefill_strided_inputs(pkg, dev):
     wide = torch.cat([q, k, v], dim=-1).to(dev)          # [T, H, 384]
     qv, kv, vv = wide[..., :DK], wide[..., DK:2 * DK], wide[..., 2 * DK:]
     bd, gd = beta.to(dev), g.to(dev)
-    out, st = pkg.call_gdn_recurrent_prefill_chunked_triton(qv, kv, vv, bd, gd)
-    out2, st2 = pkg.call_gdn_recurrent_prefill_chunked_triton(
-        qv.contiguous(), kv.contiguous(), vv.contiguous(), bd, gd)
+    run = form(pkg, which)
+    out, st = run(qv, kv, vv, bd, gd)
+    out2, st2 = run(qv.contiguous(), kv.contiguous(), vv.contiguous(), bd, gd)
     assert torch.equal(out, out2) and torch.equal(st, st2)
