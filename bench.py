@@ -950,8 +950,9 @@ def gdn_bench(pkg, dev):
         name = f"gdn_recurrent_prefill_sequential {len(lengths)} x {lengths[0]}"
         out[name] = {"us": round(ms * 1e3, 2), "tokens/s": round(T / ms * 1e3, 1),
                      "us_per_token_step": round(ms * 1e3 / max(lengths), 4)}
-    # one long prompt through the chunk-64 WY form (the runner's route for a
-    # single sequence of >= 2048 tokens), stage by stage and as the chain
+    # one long prompt alone (the runner's route for a single sequence of >= 2048
+    # tokens: segments cut for its own length; vs_sequential: against the packed
+    # batches' segments), and the chunk-64 WY ops stage by stage
     for T in (4096, 16384):
         q, k, v, beta, g = qkv(T)
         ms = time_events(lambda: pkg.call_gdn_recurrent_prefill_chunked_triton(q, k, v, beta, g), 5)

@@ -577,51 +577,49 @@ void paged_decode_split_kernel(const DecodeArgs a) {
   // there the workgroup's last wave, idle while the q rows are staged,
   // prepares both rows in LDS and writes the append.
   const bool has_new = kFused && p0 <= last_page && last_page < p1;  // uniform
-  auto stage_new = [&] {
+  [[maybe_unused]] const auto stage_new = [&] {   // the attention block's
     const int c = (lane & 31) * 8;
     u32x4_t krow = {0u, 0u, 0u, 0u};
-    if constexpr (kProlog) {
-      // RMSNorm + partial RoPE of the raw key row (both 32-lane halves compute it)
-      const u32x4_t xw = q_pre;
-      const u32x4_t ww = pi.w;
-      // chunk l (dims 8l..8l+7) pairs with chunk l +- half/8
-      const int hc = a.rope_dim / 16, l32 = lane & 31;
-      const bool first = l32 < hc, second = l32 >= hc && l32 < 2 * hc;
-      const int partner = (lane & 32) | (first ? l32 + hc : second ? l32 - hc : l32);
-      const float pf = float(seq_len - 1);  // = float(pos[b])
-      // lane j computes pair j's sine and cosine (at most 64 pairs), the lanes
-      // that rotate fetch their eight
-      float sn_j, cs_j;
-      rope_sincos(pf, pi.fq_new, sn_j, cs_j);
-      const int j0 = (first ? c : c - 8 * hc) & 63;
-      const float rs = rms_rsigma(rms_acc8(xw, 0.f), kD, a.eps);
-      float y[8];
+    // RMSNorm + partial RoPE of the raw key row (both 32-lane halves compute it)
+    const u32x4_t xw = q_pre;
+    const u32x4_t ww = pi.w;
+    // chunk l (dims 8l..8l+7) pairs with chunk l +- half/8
+    const int hc = a.rope_dim / 16, l32 = lane & 31;
+    const bool first = l32 < hc, second = l32 >= hc && l32 < 2 * hc;
+    const int partner = (lane & 32) | (first ? l32 + hc : second ? l32 - hc : l32);
+    const float pf = float(seq_len - 1);  // = float(pos[b])
+    // lane j computes pair j's sine and cosine (at most 64 pairs), the lanes
+    // that rotate fetch their eight
+    float sn_j, cs_j;
+    rope_sincos(pf, pi.fq_new, sn_j, cs_j);
+    const int j0 = (first ? c : c - 8 * hc) & 63;
+    const float rs = rms_rsigma(rms_acc8(xw, 0.f), kD, a.eps);
+    float y[8];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        y[2 * e] = round_bf16(rms_apply(bf16_lo(xw[e]), rs, bf16_lo(ww[e])));
-        y[2 * e + 1] = round_bf16(rms_apply(bf16_hi(xw[e]), rs, bf16_hi(ww[e])));
-      }
+    for (int e = 0; e < 4; ++e) {
+      y[2 * e] = round_bf16(rms_apply(bf16_lo(xw[e]), rs, bf16_lo(ww[e])));
+      y[2 * e + 1] = round_bf16(rms_apply(bf16_hi(xw[e]), rs, bf16_hi(ww[e])));
+    }
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        float o[2];
+    for (int e = 0; e < 8; e += 2) {
+      float o[2];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const float other = __shfl(y[e + u], partner);
-          const float sn = __shfl(sn_j, j0 + e + u), cs = __shfl(cs_j, j0 + e + u);
-          o[u] = y[e + u];
-          if (first || second) {
-            float o1, o2;
-            if (first) {
-              rope_rotate(y[e + u], other, cs, sn, o1, o2);
-              o[u] = o1;
-            } else {
-              rope_rotate(other, y[e + u], cs, sn, o1, o2);
-              o[u] = o2;
-            }
+      for (int u = 0; u < 2; ++u) {
+        const float other = __shfl(y[e + u], partner);
+        const float sn = __shfl(sn_j, j0 + e + u), cs = __shfl(cs_j, j0 + e + u);
+        o[u] = y[e + u];
+        if (first || second) {
+          float o1, o2;
+          if (first) {
+            rope_rotate(y[e + u], other, cs, sn, o1, o2);
+            o[u] = o1;
+          } else {
+            rope_rotate(other, y[e + u], cs, sn, o1, o2);
+            o[u] = o2;
           }
         }
-        krow[e / 2] = pack_bf16x2(o[0], o[1]);
       }
+      krow[e / 2] = pack_bf16x2(o[0], o[1]);
     }
     // Scalar page and row addresses, made opaque: the lanes' choice between
     // them must not become a vector load of either's parts, which would wait
@@ -631,7 +629,7 @@ void paged_decode_split_kernel(const DecodeArgs a) {
     global_t krow_dst = (global_t)(a.kc + phys * a.kc_p + h * a.kc_h + last_slot * a.kc_s);
     global_t vrow_dst = (global_t)(a.vc + phys * a.vc_p + h * a.vc_h + last_slot * a.vc_s);
     asm volatile("" : "+s"(krow_dst), "+s"(vrow_dst));
-    const u32x4_t vrow = kProlog ? pi.vn : ld16(vnrow + c);
+    const u32x4_t vrow = pi.vn;
     st16(lane < 32 ? &sm.kn[c] : &sm.vn[c], lane < 32 ? krow : vrow);
     *(__attribute__((address_space(1))) u32x4_t *)((lane < 32 ? krow_dst : vrow_dst) + c) =
         lane < 32 ? krow : vrow;

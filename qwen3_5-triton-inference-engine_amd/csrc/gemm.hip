@@ -1135,7 +1135,7 @@ void launch_skinny_plan(const SkinnyArgs &a, int nt, int nw, hipStream_t st) {
 // splits across workgroups, waves per workgroup.
 struct SkinnyPlan {
   int nt, blocks, split, nw;
-  int over;   // 16-column tiles past whole rounds of the CUs, left to the first workgroups
+  int over;   // 16-column tiles past one block to each CU, left to the first workgroups
 };
 // Waves per workgroup for `groups` workgroups that each cover `ks` of K: grow
 // from 4 while the grid holds fewer than 2048 waves, each wave keeps at least
@@ -1166,14 +1166,16 @@ SkinnyPlan skinny_plan(int N, int K, bool gate_up_pairs = false) {
   // Waves: enough workgroups x waves to keep the CUs streaming, each wave at
   // least one 128-wide batch of k.
   p.nw = skinny_waves(p.blocks * p.split, K / p.split);
-  // One or two blocks past whole rounds of the CUs (the GDN in_proj's 8224 =
-  // 256 x 32 + 32) go to the first workgroups, a tile each; more of them fill a
+  // One or two blocks past one to each CU (the GDN in_proj's 8224 = 256 x 32 +
+  // 32) go to the first workgroups, a tile each; more of them fill a second
   // round well enough.  Only where a wave reads its K slice in one batch
   // (K / nw = 128), so that the tile's rows are requested with the others.
-  const int past = p.blocks % 256;
+  // That is N = 8193 .. 8256 and K = 1024 on 8 waves: of this model's matrices
+  // the in_proj alone, which a decode step reads 18 times.
+  const int past = p.blocks - kCUs;
   p.over = !gate_up_pairs && p.nt == 2 && p.nw == 8 && p.split == 1 && K == 128 * p.nw &&
-                   p.blocks > 256 && past >= 1 && past <= 2
-               ? (N - (p.blocks - past) * 32 + 15) / 16
+                   (past == 1 || past == 2)
+               ? (N - kCUs * 32 + 15) / 16
                : 0;
   return p;
 }

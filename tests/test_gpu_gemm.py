@@ -288,3 +288,15 @@ def test_gemm_2d_blocks_past_a_round(pkg, dev, M, N):
     check(y, x, w)
     tail = pkg.gemm_2d(xd, wd[N - 4096:].contiguous())   # 128 blocks, no second ones
     assert torch.equal(y[:, N - 4096:], tail)
+
+
+@pytest.mark.parametrize("M", [1, 33])
+@pytest.mark.parametrize("N, K", [(16416, 1024), (8224, 1152), (8224, 512)])
+def test_gemm_2d_blocks_past_a_round_elsewhere(pkg, dev, M, N, K):
+    """A block past two rounds of the CUs and other K keep it as a workgroup of
+    its own (other waves per workgroup)."""
+    say(f"gemm_2d blocks past a round M={M} N={N} K={K}")
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).bfloat16()
+    w = (torch.randn(N, K, generator=g) * 0.05).bfloat16()
+    check(pkg.gemm_2d(x.to(dev), w.to(dev)), x, w)
