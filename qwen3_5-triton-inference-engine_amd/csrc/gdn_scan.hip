@@ -683,7 +683,7 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
   };
 
   if (tid == 0) L.wild = 0;
-  bool wild = false;   // this wavefront met a value that is not finite
+  uint64_t wild = 0;   // not 0: this wavefront met a value that is not finite
   // the block of T above the diagonal is zero and never written again
   for (int i = tid; i < 2 * 3 * 16 * 4; i += 256)
     *reinterpret_cast<u32x2_t *>(&L.T[i / 192][i / 64 % 3][i / 4 % 16][16 + 4 * (i % 4)]) =
@@ -990,7 +990,7 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
       int t_bad = kC;
       const bool any = __ballot(!(fabsf(delta[15]) <= kMaxFinite) && hf == 1) != 0;
       if (any) {
-        wild = true;
+        wild = 1;
 #pragma unroll
         for (int r = 15; r >= 0; --r)
           if (!(fabsf(R[r]) <= kMaxFinite)) t_bad = (r & 3) + 8 * (r >> 2) + 4 * hf;
@@ -1004,7 +1004,7 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
       if constexpr (!kState) {
         const f32x16_t o = apply(L.A[cc], Ao, delta, lr, hf, qs);
         // (row 31 of this product sees every row of delta)
-        wild |= __ballot(!(fabsf(o[15]) <= kMaxFinite) && hf == 1) != 0;
+        wild |= __ballot(!(fabsf(o[15]) <= kMaxFinite));
         bf16_t *op = a.out + tb * a.o_t + h * a.o_h;
         const int pitch = opaque(int(a.o_t) * 2);
         const auto rs = rows_rsrc(op, pitch, nv, a.dv * 2);
@@ -1095,9 +1095,9 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
     for (int r = 0; r < 16; ++r)
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) z[rt] = __fmaf_rn(S[rt][r], 0.f, z[rt]);
-    wild |= __ballot((z[0] + z[1]) + (z[2] + z[3]) != 0.f) != 0;
-    if (t_lo < t_hi) wild |= __builtin_amdgcn_readfirstlane(L.wild) != 0;
-    if (wild) {
+    wild |= __ballot((z[0] + z[1]) + (z[2] + z[3]) != 0.f);
+    if (t_lo < t_hi) wild |= uint64_t(__builtin_amdgcn_readfirstlane(L.wild));
+    if (wild != 0) {
       __threadfence_block();   // other lanes' results are read back
       walk_not_finite<kContig, 8>(args_again(), s0, t_lo, t_hi, h, vb * 128 + wave * kWCols,
                                   lane_again(), dst);
