@@ -48,11 +48,12 @@
 // (cutting fp32 values is most of them) per wavefront, and T's chain (~4000
 // cycles per group) holds up the workgroup's four; two workgroups per CU fill
 // one another's gaps (LDS and 256 VGPRs allow no third).  Measured (16 heads,
-// recurrence alone, against one wavefront per 16 columns walking token by
-// token): 32 x 128 tokens 200 -> 43 us, 24 prompts of 22..4096 tokens (23.8k)
-// 3.10 ms -> 0.47 ms, one prompt of 1000 tokens 304 -> 142 us, one of 5003
-// 287 (chunk ops of csrc/gdn_chunk.hip) -> 189 us; one of 9 to 16 tokens 6.4 to
-// 8.6 -> 9.5 us, the chunk's fixed cost.
+// recurrence alone, against the walk of whole sequences token by token): 32 x
+// 128 tokens 188 -> 42 us (48 where the longest sequence is not known), 24
+// prompts of 22..4096 tokens (23772) 2.09 -> 0.51 ms, a packed batch of one
+// sequence of 1000 tokens 308 -> 145 us, one prompt of 5003 alone 278 (chunk
+// ops of csrc/gdn_chunk.hip) -> 181 us; one of 9 to 16 tokens 6.4 to 8.6 -> 9.5
+// us, the chunk's fixed cost.
 #include "gdn_common.h"
 
 using namespace wy;
@@ -64,8 +65,10 @@ constexpr int kC = 32;        // tokens per chunk
 constexpr int kG = 64;        // tokens staged together (two chunks)
 // Tokens per segment of a packed batch.  Shorter ones fill the chip when few
 // sequences are there, longer ones save walking twice what fills it anyway: 128
-// / 256 / 512 / 1024 tokens: 24 prompts of 22..4096 tokens 710 / 557 / 470 / 402
-// us, one of 5003 250 / 194 / 189 / 288, one of 1000 68 / 85 / 142 / 153.
+// / 256 / 512 / 1024 tokens: 24 prompts of 22..4096 tokens 755 / 579 / 512 / 422
+// us, 32 of 600 489 / 400 / 396 / 191, one of 5003 269 / 213 / 206 / 293, one of
+// 1000 77 / 92 / 146 / 155.  One length for every sequence is a compromise of
+// these.
 #ifndef WY_GDN_SEG
 #define WY_GDN_SEG 512
 #endif

@@ -39,6 +39,8 @@ constexpr int kMaxSplit = 4;  // K splits across workgroups (skinny kernel)
 //      to xout (the residual stream);
 //   2: A = swiglu(x[:, :K], x[:, up_off:up_off+K]) = bf16(up * gate * sigmoid(gate)).
 // Each equals the standalone kernels followed by the plain GEMM bit for bit.
+// 1 and 2 serve the ops rmsnorm_gemm_2d and swiglu_gemm_2d; the model's decode
+// step, where separate launches are faster at every batch, uses 0.
 struct ProArgs {
   const bf16_t *res;
   int64_t res0;
