@@ -40,9 +40,10 @@
 // Values that are not finite (infinities and NaN in the inputs, sums past
 // FLT_MAX): the products spread them further than the recurrence does, and a
 // cut infinity is NaN.  They are kept out of earlier tokens' and other
-// columns' results, and a wavefront that met one walks its columns once more
-// token by token, putting the recurrence's own value wherever its output or
-// state is not finite.
+// columns' results, and a wavefront that met an infinity walks its columns once
+// more token by token, putting the recurrence's own value wherever its output or
+// state is not finite.  (A NaN needs no walk; a segment behind the one of the
+// infinity gets NaN.)
 //
 // What bounds it: a chunk is 96 MFMAs of 32 cycles and ~750 VALU operations
 // (cutting fp32 values is most of them) per wavefront, and T's chain (~4000
@@ -109,7 +110,7 @@ struct ScanLds {
                               // zero one
   float Gh[kG], Gl[kG], beta[kG];
   float eG[kG], E[kG], eL[4];
-  int wild;   // a value of A was not finite
+  int wild;   // an infinity in L, A, k, q, beta or g
 };
 static_assert(sizeof(ScanLds) <= 80 * 1024, "two workgroups per CU");
 static_assert(offsetof(ScanLds, T) % 16 == 0 && offsetof(ScanLds, A) % 16 == 0 &&
@@ -443,13 +444,16 @@ __device__ __forceinline__ void step_scaled(float (&s)[kRows][NC], float &c, con
     for (int j = 0; j < NC; ++j) s[i][j] = __fmaf_rn(k[i], dsc[j], s[i][j]);
 }
 
-// A whole sequence from a zero state, the wavefront's 4 NC columns from col0.
-// The sums keep one order whatever NC is: the same bits.  kAhead tokens are in flight: every load and store is
-// unconditional (a request past the end re-reads the last token, the 16 lanes of
-// a row store the same output), so a wait names exactly the token a step needs.
-template <bool kContig, int NC>
-__device__ __forceinline__ void walk(const GdnArgs &a, int s0, int len, int b, int h, int col0,
-                                     int lane) {
+// Tokens [0, len) of the sequence at s0 from a zero state, the wavefront's 4 NC
+// columns from col0; the state goes to sp (null: nowhere).  The sums keep one
+// order whatever NC is: the same bits.  kAhead tokens are in flight: every load
+// and store is unconditional (a request past the end re-reads the last token, the
+// 16 lanes of a row store the same output), so a wait names exactly the token a
+// step needs.
+// kMend: only what is there and not finite is replaced, outputs from t_lo on.
+template <bool kContig, int NC, bool kMend = false>
+__device__ __forceinline__ void walk(const GdnArgs &a, int s0, int len, int h, int col0, int lane,
+                                     float *sp, int t_lo = 0) {
   constexpr int kAhead = NC == 1 ? 4 : 2;
   const int kg = lane & 15, col = col0 + NC * (lane >> 4);
   float s[kRows][NC], c = 1.f;
@@ -460,7 +464,12 @@ __device__ __forceinline__ void walk(const GdnArgs &a, int s0, int len, int b, i
   if (len > 0) {
     auto put = [&](int t, const float (&o)[NC]) {
       bf16_t *op = a.out + int64_t(s0 + t) * a.o_t + h * a.o_h + col * a.o_d;
-      if constexpr (!kContig || NC == 1) {
+      if constexpr (kMend) {
+        if (t < t_lo) return;
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+          if ((op[j * a.o_d] & 0x7f80) == 0x7f80) op[j * a.o_d] = bf16_t(f32_to_bf16_bits(o[j]));
+      } else if constexpr (!kContig || NC == 1) {
 #pragma unroll
         for (int j = 0; j < NC; ++j) op[j * a.o_d] = bf16_t(f32_to_bf16_bits(o[j]));
       } else {
@@ -492,11 +501,13 @@ __device__ __forceinline__ void walk(const GdnArgs &a, int s0, int len, int b, i
         put(whole + u, o);
       }
   }
-  float *sp = a.state + b * a.s_b + h * a.s_h + int64_t(kg * kRows) * a.s_k + col;
+  if (kMend && sp == nullptr) return;
+  sp += int64_t(kg * kRows) * a.s_k + col;
 #pragma unroll
   for (int i = 0; i < kRows; ++i)
 #pragma unroll
-    for (int j = 0; j < NC; ++j) sp[i * a.s_k + j] = c * s[i][j];
+    for (int j = 0; j < NC; ++j)
+      if (!kMend || !(fabsf(sp[i * a.s_k + j]) <= kMaxFinite)) sp[i * a.s_k + j] = c * s[i][j];
 }
 
 // A batch of sequences of at most kWalk tokens each: one wavefront to 4 NC
@@ -507,42 +518,26 @@ __global__ __launch_bounds__(64) void gdn_walk_kernel(const GdnArgs a, int token
   const int h = (blockIdx.x / batch) % a.heads;
   const int col0 = blockIdx.x / (batch * a.heads) * 4 * NC;
   const int s0 = seq_start(a.cu_seqlens, token_num, b);
-  walk<kContig, NC>(a, s0, seq_start(a.cu_seqlens, token_num, b + 1) - s0, b, h, col0,
-                    threadIdx.x);
+  walk<kContig, NC>(a, s0, seq_start(a.cu_seqlens, token_num, b + 1) - s0, h, col0, threadIdx.x,
+                    a.state + b * a.s_b + h * a.s_h);
 }
 
-// The wavefront's 4 NC columns from col0 over tokens [0, t_hi) of the sequence
-// at s0.  Where the chunks' output from token t_lo on, or the
-// state they left at sp (null: not the last segment), is not finite, the
-// walk's takes its place.
-template <bool kContig, int NC>
-__device__ __forceinline__ void walk_not_finite(const GdnArgs &a, int s0, int t_lo, int t_hi,
-                                                int h, int col0, int lane, float *sp) {
-  const int kg = lane & 15, col = col0 + NC * (lane >> 4);
-  float s[kRows][NC], c = 1.f;
+// ---- infinities.  (fmaxf passes NaN by.)
+__device__ __forceinline__ bool has_inf(const f32x16_t &v) {
+  float m = 0.f;
 #pragma unroll
-  for (int i = 0; i < kRows; ++i)
-#pragma unroll
-    for (int j = 0; j < NC; ++j) s[i][j] = 0.f;
-  for (int t = 0; t < t_hi; ++t) {
-    TokenRaw<NC> in;
-    load_token_raw<kContig, NC>(a, s0 + t, h, kg, col, in);
-    float o[NC];
-    step_scaled<NC>(s, c, in, o);
-    if (t < t_lo) continue;
-    bf16_t *op = a.out + int64_t(s0 + t) * a.o_t + h * a.o_h + col * a.o_d;
-#pragma unroll
-    for (int j = 0; j < NC; ++j)
-      if ((op[j * a.o_d] & 0x7f80) == 0x7f80) op[j * a.o_d] = bf16_t(f32_to_bf16_bits(o[j]));
-  }
-  if (sp == nullptr) return;
-#pragma unroll
-  for (int i = 0; i < kRows; ++i)
-#pragma unroll
-    for (int j = 0; j < NC; ++j) {
-      float *p = sp + (kg * kRows + i) * a.s_k + col + j;
-      if (!(fabsf(*p) <= kMaxFinite)) *p = c * s[i][j];
-    }
+  for (int r = 0; r < 16; ++r) m = fmaxf(m, fabsf(v[r]));
+  return m > kMaxFinite;
+}
+__device__ __forceinline__ bool has_inf(const f32x16_t (&S)[4]) {
+  return has_inf(S[0]) || has_inf(S[1]) || has_inf(S[2]) || has_inf(S[3]);
+}
+// one in keys 64 hf .. + 63 of a row of k or q
+__device__ __forceinline__ bool row_has_inf(const bf16_t *row, int hf) {
+  int found = 0;
+#pragma unroll 1
+  for (int i = 64 * hf; i < 64 * hf + 64; ++i) found |= (row[i] & 0x7fff) == 0x7f80;
+  return found != 0;
 }
 
 // kState: a non-last segment's state (and homogeneous solution) only.
@@ -586,7 +581,9 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
   const int len = seq_start(a.cu_seqlens, token_num, b + 1) - s0;
   if constexpr (!kState) {
     if (len <= kWalk) {
-      walk<kContig, 8>(args_again(), s0, len, b, h, vb * 128 + wave * kWCols, lane_again());
+      const GdnArgs ar = args_again();
+      walk<kContig, 8>(ar, s0, len, h, vb * 128 + wave * kWCols, lane_again(),
+                       ar.state + b * ar.s_b + h * ar.s_h);
       return;
     }
   }
@@ -685,8 +682,8 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
     *reinterpret_cast<u32x2_t *>(&dst[row][kslot + 8]) = u32x2_t{x[2], x[3]};
   };
 
-  if (tid == 0) L.wild = 0;
-  uint64_t wild = 0;   // not 0: this wavefront met a value that is not finite
+  if (tid == 192) L.wild = 0;   // (wave 3 is the first to set it)
+  uint64_t wild = 0;   // not 0: this wavefront met an infinity
   // the block of T above the diagonal is zero and never written again
   for (int i = tid; i < 2 * 3 * 16 * 4; i += 256)
     *reinterpret_cast<u32x2_t *>(&L.T[i / 192][i / 64 % 3][i / 4 % 16][16 + 4 * (i % 4)]) =
@@ -747,6 +744,8 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
       // a beta that is not finite makes its row of v - k S (through eG) not
       // finite, and so the columns from this token on; T itself stays finite
       const bool fine = fabsf(rb) <= kMaxFinite;
+      if (!kState && __ballot(lane < nval && (fabsf(rb) > kMaxFinite || rg > kMaxFinite)) != 0)
+        L.wild = 1;
       L.beta[lane] = lane < nval && fine ? rb : 0.f;
       L.eG[lane] = lane >= nval || fine ? __builtin_amdgcn_exp2f(gh) : __builtin_nanf("");
       L.E[lane] = __builtin_amdgcn_exp2f(float(Gl - G));
@@ -802,11 +801,17 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
           }
           if (__ballot(!(fabsf(nans) <= kMaxFinite)) != 0) {
             // as for beta: mark the rows of L that are not finite, keep T finite
-            for (int i = 0; i < kC; ++i)
-              if (!(fabsf(Lt[lr * kLP + i]) <= kMaxFinite)) {
+            bool inf = !kState && row_has_inf(L.K[rb0 + lr], hf);
+#pragma unroll 1
+            for (int i = 0; i < kC; ++i) {
+              const float x = Lt[lr * kLP + i];
+              if (!(fabsf(x) <= kMaxFinite)) {
+                inf |= fabsf(x) > kMaxFinite;
                 L.eG[rb0 + i] = __builtin_nanf("");
                 Lt[lr * kLP + i] = 0.f;
               }
+            }
+            if (!kState && __ballot(inf) != 0) L.wild = 1;
           }
           // T = (I + L)^-1 diag(beta).  The two diagonal 16 x 16 blocks by
           // back substitution of x (I + L) = e_t, a row t per lane (the upper
@@ -881,7 +886,12 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
 #pragma unroll
             for (int n = 0; n < 3; ++n) st16(&L.A[cc][n][lr][16 * s + 8 * hf], p.p[n]);
           }
-          if (__ballot(!(fabsf(nans) <= kMaxFinite)) != 0) L.wild = 1;
+          if (__ballot(!(fabsf(nans) <= kMaxFinite)) != 0) {
+            bool inf = row_has_inf(L.K[rb0 + lr], hf) || row_has_inf(L.Q[rb0 + lr], hf);
+#pragma unroll 1
+            for (int i = 0; i < kC; ++i) inf |= (L.A[cc][0][lr][i] & 0x7fff) == 0x7f80;
+            if (__ballot(inf) != 0) L.wild = 1;
+          }
         }
       }
     }
@@ -988,12 +998,12 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
       // Row 31 of the product sees every row of R: where it is not finite, a
       // value that is not finite sits in this column of R from some token
       // t_bad on, and 0 x inf has spread it to the rows before as well.  Those
-      // are formed again without it; from t_bad on the column is set to NaN,
-      // which the walk at the end replaces.
+      // are formed again without it; from t_bad on the column is set to NaN
+      // (which the walk at the end replaces if it came from an infinity).
       int t_bad = kC;
       const bool any = __ballot(!(fabsf(delta[15]) <= kMaxFinite) && hf == 1) != 0;
       if (any) {
-        wild = 1;
+        if constexpr (!kState) wild |= __ballot(has_inf(R) || has_inf(S));
 #pragma unroll
         for (int r = 15; r >= 0; --r)
           if (!(fabsf(R[r]) <= kMaxFinite)) t_bad = (r & 3) + 8 * (r >> 2) + 4 * hf;
@@ -1007,7 +1017,8 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
       if constexpr (!kState) {
         const f32x16_t o = apply(L.A[cc], Ao, delta, lr, hf, qs);
         // (row 31 of this product sees every row of delta)
-        wild |= __ballot(!(fabsf(o[15]) <= kMaxFinite));
+        if (__ballot(!(fabsf(o[15]) <= kMaxFinite)) != 0)
+          wild |= __ballot(has_inf(o) || has_inf(delta) || has_inf(S));
         bf16_t *op = a.out + tb * a.o_t + h * a.o_h;
         const int pitch = opaque(int(a.o_t) * 2);
         const auto rs = rows_rsrc(op, pitch, nv, a.dv * 2);
@@ -1098,12 +1109,12 @@ __global__ __launch_bounds__(256, 2) void gdn_scan_kernel(const GdnArgs a, int t
     for (int r = 0; r < 16; ++r)
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) z[rt] = __fmaf_rn(S[rt][r], 0.f, z[rt]);
-    wild |= __ballot((z[0] + z[1]) + (z[2] + z[3]) != 0.f);
+    if (__ballot((z[0] + z[1]) + (z[2] + z[3]) != 0.f) != 0) wild |= __ballot(has_inf(S));
     if (t_lo < t_hi) wild |= uint64_t(__builtin_amdgcn_readfirstlane(L.wild));
     if (wild != 0) {
       __threadfence_block();   // other lanes' results are read back
-      walk_not_finite<kContig, 8>(args_again(), s0, t_lo, t_hi, h, vb * 128 + wave * kWCols,
-                                  lane_again(), dst);
+      walk<kContig, 8, true>(args_again(), s0, t_hi, h, vb * 128 + wave * kWCols, lane_again(), dst,
+                             t_lo);
     }
   }
 }
