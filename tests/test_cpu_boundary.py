@@ -526,3 +526,29 @@ def test_host_tensors_never_reach_a_launch(pkg, monkeypatch):
             q, q, v, beta, beta, torch.tensor([0, 8], dtype=torch.int32),
             torch.zeros(1, 2, 128, 128))
     assert not calls
+
+
+def test_gdn_prefill_forms_reject_before_launch(pkg):
+    """The packed prefill with a known longest length and the prompt alone
+    refuse shapes, NULL tables, short or misaligned workspaces before a launch."""
+    lib = pkg._lib.load()
+    d, odd = ctypes.c_void_p(256), ctypes.c_void_p(260)
+    s3 = (ctypes.c_int64 * 3)(2048, 128, 1)
+    s2 = (ctypes.c_int64 * 2)(16, 1)
+    s4 = (ctypes.c_int64 * 4)(16 * 128 * 128, 128 * 128, 128, 1)
+    base = [d, s3, d, s3, d, s3, d, s2, d, s2, d, s3, d, s4]
+    packed, prompt = lib.wy_gdn_prefill_varlen_max, lib.wy_gdn_prefill_prompt
+    assert packed(*base, None, 2048, 0, 2, 16, 128, 128, None, 0, None) == -1
+    assert packed(*base, d, 2048, -1, 2, 16, 128, 128, None, 0, None) == -2
+    assert packed(*base, d, 2048, 0, 0, 16, 128, 128, None, 0, None) == 0    # nothing to do
+    assert packed(*base, d, 2048, 0, 2, 16, 64, 128, None, 0, None) == -4
+    need = lib.wy_gdn_prefill_varlen_workspace_bytes(2048, 16, 128)
+    assert need > 0 and lib.wy_gdn_prefill_varlen_workspace_bytes(512, 16, 128) == 0
+    assert packed(*base, d, 2048, 0, 2, 16, 128, 128, d, need - 1, None) == -5
+    assert packed(*base, d, 2048, 0, 2, 16, 128, 128, odd, need, None) == -3
+    assert prompt(*base, 0, 16, 128, 128, None, 0, None) == -2
+    assert prompt(*base, 300, 16, 128, 96, None, 0, None) == -4
+    need = lib.wy_gdn_prefill_prompt_workspace_bytes(300, 16, 128)
+    assert need > 0 and lib.wy_gdn_prefill_prompt_workspace_bytes(192, 16, 128) == 0
+    assert prompt(*base, 300, 16, 128, 128, d, need - 1, None) == -5
+    assert prompt(*base, 300, 16, 128, 128, odd, need, None) == -3

@@ -101,6 +101,31 @@ def test_short_sequences_same_bits_by_every_route(pkg, dev, lens):
     assert rel(out[rows], o64) < 2 ** -9 and rel(st[some], s64) < 1e-6
 
 
+def test_short_sequences_other_strides_and_two_column_blocks(pkg, dev):
+    """Walked sequences beside long ones: other strides, and 256 value columns,
+    give the bits of contiguous inputs and of each half of the columns alone."""
+    lens = [8, 9, 0, 1, 40, SEG + 5]
+    T = sum(lens)
+    q, k, v, beta, g = inputs(T, dev, 29, 0.1)
+    cu = cu_of(lens, dev)
+    want = pkg.gdn_recurrent_prefill_sequential(q, k, v, beta, g, cu)
+    wide = torch.zeros(T, H, 2 * D, dtype=v.dtype, device=dev)
+    wide[..., ::2] = v
+    got = pkg.gdn_recurrent_prefill_sequential(q, k, wide[..., ::2], beta, g, cu)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    v2 = torch.cat([v, v.flip(0)], -1)
+    out, st = pkg.gdn_recurrent_prefill_sequential(q, k, v2, beta, g, cu)
+    half = pkg.gdn_recurrent_prefill_sequential(q, k, v.flip(0).contiguous(), beta, g, cu)
+    for i, (o, s) in enumerate((want, half)):
+        assert torch.equal(out[..., i * D:(i + 1) * D], o)
+        assert torch.equal(st[..., i * D:(i + 1) * D], s)
+    prompt = pkg.call_gdn_recurrent_prefill_chunked_triton
+    for n in (5, 400):
+        o2, s2 = prompt(*(x[:n] for x in (q, k, v2, beta, g)))
+        o1, s1 = prompt(*(x[:n] for x in (q, k, v, beta, g)))
+        assert torch.equal(o2[..., :D], o1) and torch.equal(s2[..., :D], s1)
+
+
 # one prompt alone: walked, in one piece, at the first cut, a segment's edges
 @pytest.mark.parametrize("T", [1, 8, 9, 64, 192, 193, 256, 257, 1024, 1025, 2100])
 def test_prompt_alone_vs_recurrence(pkg, dev, T):
